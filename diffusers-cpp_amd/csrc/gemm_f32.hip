@@ -1,29 +1,45 @@
 // gemm_f32.hip -- fp32 Linear and attention for graphs whose weights and
 // activations are both F32, the reference's own precision (Linear::forward ->
 // Runtime::mul_mat with F32 weights, src/nn/Linear.cpp:17-36; ggml computes
-// such products in fp32), on the fp32 matrix cores of gfx950
-// (v_mfma_f32_32x32x2_f32: products and sums in fp32).
+// such products in fp32).
 //
 // GEMM: C[m][n] = sum_k A[m][k] * B[n][k] (+ bias[n]) (+ D[m][n]), A the
-// activation [M, K] and B the weight [N, K], both K-contiguous.  A workgroup
-// of four waves computes a 128 x 128 tile, each wave 64 x 64 (2 x 2 blocks of
-// 32 x 32), through K chunks of 16 staged in LDS (register-staged, double
-// buffered).  As in the bf16 kernels the MFMA computes C^T = B A^T: the
-// weight rows are the instruction's A operand, the activation rows its B
-// operand, so lane l holds C[m = l % 32][n = 8 (i / 4) + 4 (l / 32) + i % 4]
-// of each block and stores 4 consecutive n.  MFMA s of a chunk (s = 0..7)
-// multiplies the k-pair {s, 8 + s}: lanes 0-31 supply k = s and lanes 32-63
-// k = 8 + s, so each lane reads its 8 k of a row as two 16-byte LDS loads.
-// The sum is blocked in two levels: MFMA s accumulates into set s % 2 of two
-// running sets, and every 8 chunks (128 k) the two sets are added, (set 0 +
-// set 1), into the tile's total and cleared.  A running set then adds at most
-// 32 MFMA results of small partial sums and the total K/128 block sums, so
-// fp32 rounding grows over about 32 + K/128 additions instead of K/2 for one
-// chain (at K = 12288 one chain drifted 1.8e-5 from the fp64 sum, four sets
-// of K/8 additions 1.0e-5), and the two sets' chains are independent, so an
-// MFMA rarely waits on the previous one's result.
+// activation [M, K] and B the weight [N, K], both K-contiguous.  The fp32
+// matrix cores (157 TFLOP/s) bound this product, the bf16 ones (2.5 PFLOP/s)
+// do not: each operand is split exactly into three bf16 parts, x = x0 + x1 +
+// x2 (8 + 8 + 8 bits, each the rounded remainder of the last), and the product
+// taken as the six bf16 MFMAs x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0 with
+// fp32 accumulation.  The three left out are below 2^-26 of |x w|, under fp32's
+// own rounding of one product.  x0 w0 is summed by itself, in runs of 128 k
+// that are then added to the tile's total, and the five small ones in an
+// accumulator of their own, whose rounding is 2^-8 of the other's; so the sum
+// is rounded about 8 + K/128 times where the fp32 MFMA's was 64 + K/128.
+// Relative error against 64 bits (2-norm, N(0, 1) x N(0, 0.02)), fp32 MFMAs ->
+// here: K = 64 1.04e-7 -> 5.0e-8, 256 1.50e-7 -> 7.1e-8, 3072 1.74e-7 ->
+// 1.14e-7, 12288 2.32e-7 -> 1.91e-7.  Time at 1536 x 27648 x 3072: 3761 us (69
+// TFLOP/s) -> 1472 us (177); 1536 x 3072 x 9216: 2023 -> 647 us.
+//
+// A workgroup of four waves computes a 128 x 128 tile, each wave 64 x 64 (2 x 2
+// blocks of 32 x 32; three sets of 64 accumulators leave room for two waves
+// per SIMD), through chunks of 16 k in three LDS stages.  Both operands are
+// loaded into registers, split there (5.5 VALU instructions an element) and
+// written to LDS as three planes, so each element is split once per workgroup
+// and each plane read feeds two MFMAs of three products.  Chunk kt + 2 is split
+// and chunk kt + 3 loaded while chunk kt is multiplied.  The waves run their
+// MFMAs at raised priority (s_setprio), so of a SIMD's two waves one keeps
+// the matrix core while the other splits: 1801 -> 1501 us at 1536 x 27648 x
+// 3072.  A larger wave tile does not fit the registers; running sums without
+// the separate small accumulator do (156 TFLOP/s before the priorities against
+// 148), but were 10% less exact than the fp32 MFMAs.
+// As in the bf16 kernels the MFMA computes C^T = B A^T: the weight rows are the
+// instruction's A operand, the activation rows its B operand, so lane l holds
+// C[m = l % 32][n = 8 (i / 4) + 4 (l / 32) + i % 4] of each block and stores 4
+// consecutive n.
 // Rows past M or N load a clamped valid row (products never stored); k past
 // K loads zeros, so any K >= 1 is exact.
+// Operands outside the split's range (not finite, above 2^30, or so small that
+// a part of them falls below bf16's range and it would show) send their tile
+// through the fp32 matrix cores instead (f32_tile_native).
 //
 // Attention (no mask, head_dim 128): per (batch, head), S = Q K^T by the
 // GEMM, P = softmax(scale S) row by row in fp32 (max, then expf(scale s - max),
@@ -37,11 +53,13 @@
 namespace dit {
 namespace {
 
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kF32MaxGroup = 8;
 constexpr int FT = 128;          // tile edge
 constexpr int FKC = 16;          // K per chunk
+constexpr int FLUSH = 8;         // chunks per run of the sum
 constexpr int FKP = FKC + 4;     // padded LDS row, floats (80 bytes: 16 lanes' 16-byte reads hit distinct banks)
 
 struct F32Problem {
@@ -52,7 +70,7 @@ struct F32Problem {
     const float* bias;
     int64_t lda, ldb, ldc, ldd;
     int M, N, K;
-    int vec;  // 16-byte row loads allowed (K % 16 == 0, lda, ldb % 4 == 0, A and B 16-byte aligned)
+    int vec;  // 16-byte row loads allowed (f32_validate)
 };
 
 struct F32Group {
@@ -61,8 +79,12 @@ struct F32Group {
     int count;
 };
 
-// This workgroup's problem and tile; XCD-contiguous numbering as in the bf16
-// GEMM (each of the 8 XCDs takes a contiguous range of tiles).
+// This workgroup's problem and tile; XCD-contiguous numbering (each of the 8
+// XCDs takes a contiguous range of tiles), in groups of 8 tile rows that share
+// their weight columns: 1536 x 27648 x 3072 took 1524 us row by row, 1482 in
+// groups of 4, 1472 of 8, 1458 of 16 (one group); 1536 x 3072 x 9216 665, 660,
+// 647 and 660.
+constexpr int F32_GROUP_M = 8;
 __device__ __forceinline__ const F32Problem& f32_locate(const F32Group& g, int* tm, int* tn) {
     uint32_t bid = blockIdx.x;
     const uint32_t nb = gridDim.x, q = nb >> 3;
@@ -71,127 +93,287 @@ __device__ __forceinline__ const F32Problem& f32_locate(const F32Group& g, int* 
     while (pi + 1 < g.count && (int)bid >= g.tile_start[pi + 1]) ++pi;
     const F32Problem& p = g.p[pi];
     const int local = (int)bid - g.tile_start[pi];
-    const int tiles_n = (p.N + FT - 1) / FT;
-    *tm = local / tiles_n;
-    *tn = local - *tm * tiles_n;
+    const int tiles_m = (p.M + FT - 1) / FT, tiles_n = (p.N + FT - 1) / FT;
+    const int per_group = F32_GROUP_M * tiles_n;
+    const int group = local / per_group, first_m = group * F32_GROUP_M;
+    const int rows = min(tiles_m - first_m, F32_GROUP_M);
+    const int in_group = local - group * per_group;
+    *tm = first_m + in_group % rows;
+    *tn = in_group / rows;
     return p;
 }
 
-// 8 consecutive k of one row from k0, zeros past K.
-__device__ __forceinline__ void load8(const float* row, int k0, int K, bool vec, float4& lo, float4& hi) {
-    if (vec) {
-        lo = *reinterpret_cast<const float4*>(row + k0);
-        hi = *reinterpret_cast<const float4*>(row + k0 + 4);
-        return;
-    }
-    float v[8];
+// 4 consecutive k of one row from k0, zeros past K.
+template <bool VEC>
+__device__ __forceinline__ float4 load4(const float* row, int k0, int K) {
+    if constexpr (VEC) return *reinterpret_cast<const float4*>(row + k0);
+    float v[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = k0 + e < K ? row[k0 + e] : 0.0f;
-    lo = make_float4(v[0], v[1], v[2], v[3]);
-    hi = make_float4(v[4], v[5], v[6], v[7]);
+    for (int e = 0; e < 4; ++e) v[e] = k0 + e < K ? row[k0 + e] : 0.0f;
+    return make_float4(v[0], v[1], v[2], v[3]);
 }
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const F32Group grp) {
-    constexpr int FM = 2, FN = 2;
-    __shared__ __attribute__((aligned(16))) float sa[2][FT * FKP];
-    __shared__ __attribute__((aligned(16))) float sb[2][FT * FKP];
+// 4 fp32 as three planes of 4 bf16 (8 bytes each), x = p0 + p1 + p2.
+__device__ __forceinline__ void split3(const float4& x, uint2 (&p)[3]) {
+    const uint32_t h0 = pack_bf16x2(x.x, x.y), h1 = pack_bf16x2(x.z, x.w);
+    const float r0 = x.x - bf16_lo(h0), r1 = x.y - bf16_hi(h0), r2 = x.z - bf16_lo(h1), r3 = x.w - bf16_hi(h1);
+    const uint32_t m0 = pack_bf16x2(r0, r1), m1 = pack_bf16x2(r2, r3);
+    p[0] = make_uint2(h0, h1);
+    p[1] = make_uint2(m0, m1);
+    p[2] = make_uint2(pack_bf16x2(r0 - bf16_lo(m0), r1 - bf16_hi(m0)), pack_bf16x2(r2 - bf16_lo(m1), r3 - bf16_hi(m1)));
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// max(m, |a|, |b|) in one instruction (fmaxf quiets each operand first); a NaN
+// is passed over.
+__device__ __forceinline__ float max3_abs(float m, float a, float b) {
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
+    return m;
+}
+
+// A stage: 16 k of the A rows, then of the B rows, as three planes of 256 rows
+// x 32 bytes; half h (8 k) of row r at half h ^ xswz(r), so that 8 (32-bank) or
+// 16 (64-bank) consecutive rows at one half hit distinct banks.
+constexpr int XPLANE = 2 * FT * FKC * 2, XSTAGE = 3 * XPLANE, XSTAGES = 3;
+__device__ __forceinline__ int xswz(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
+// Largest |operand| and smallest |sum| the split products are used for.
+constexpr float kSplitMax = 1073741824.0f;  // 2^30
+constexpr float kSplitMin = 8.8817841970012523e-16f;  // 2^-50
+constexpr float kTiny = 2.9103830456733704e-11f;  // 2^-35
+
+// The tile on the fp32 matrix cores (v_mfma_f32_32x32x2_f32): products and
+// sums in fp32 for operands of any magnitude.  Chunks of 16 k; MFMA s of a
+// chunk (s = 0..7) multiplies the k-pair {s, 8 + s}: lanes 0-31 supply k = s
+// and lanes 32-63 k = 8 + s, into set s % 2 of two running sums; runs of 8 chunks
+// are summed (set 0 + set 1) before they join the tile's total.
+template <bool VEC>
+__device__ __forceinline__ void f32_tile_native(const F32Problem& p, uint8_t* smem, int m0, int n0, int wm, int wn,
+                                                f32x16_t (&tot)[2][2]) {
+    constexpr int OP = FT * FKP;
+    float* sm = reinterpret_cast<float*>(smem);  // [A | B][128][FKP]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int row = tid >> 1, kh = (tid & 1) * 8;
+    const float* arow = p.A + (int64_t)min(m0 + row, p.M - 1) * p.lda + kh;
+    const float* brow = p.B + (int64_t)min(n0 + row, p.N - 1) * p.ldb + kh;
+    f32x16_t acc[2][2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[0][j][i][e] = acc[1][j][i][e] = tot[j][i][e] = 0.f;
+    const int lrow = lane & 31, lk = (lane >> 5) * 8;
+    const int nk = (p.K + FKC - 1) / FKC;
+    for (int kt = 0; kt < nk; ++kt) {
+        const int k0 = kt * FKC, kn = p.K - kh;
+        const float4 a0 = load4<VEC>(arow, k0, kn), a1 = load4<VEC>(arow, k0 + 4, kn);
+        const float4 b0 = load4<VEC>(brow, k0, kn), b1 = load4<VEC>(brow, k0 + 4, kn);
+        __syncthreads();  // every wave's reads of the previous chunk are done
+        float* a = sm + row * FKP + kh;
+        *reinterpret_cast<float4*>(a) = a0;
+        *reinterpret_cast<float4*>(a + 4) = a1;
+        *reinterpret_cast<float4*>(a + OP) = b0;
+        *reinterpret_cast<float4*>(a + OP + 4) = b1;
+        __syncthreads();
+#pragma unroll
+        for (int st = 0; st < 8; ++st) {
+            float w[2], x[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                w[j] = sm[OP + (wn + 32 * j + lrow) * FKP + lk + st];
+                x[j] = sm[(wm + 32 * j + lrow) * FKP + lk + st];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[st & 1][j][i] =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(w[j], x[i], acc[st & 1][j][i], 0, 0, 0);
+        }
+        if ((kt + 1) % FLUSH == 0 || kt + 1 == nk) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        tot[j][i][e] += acc[0][j][i][e] + acc[1][j][i][e];
+                        acc[0][j][i][e] = acc[1][j][i][e] = 0.f;
+                    }
+        }
+    }
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[XSTAGES * XSTAGE];
+    static_assert(2 * FT * FKP * 4 <= XSTAGES * XSTAGE, "the fp32 tile's stage");
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tm, tn;
     const F32Problem& p = f32_locate(grp, &tm, &tn);
     const int m0 = tm * FT, n0 = tn * FT;
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const bool vec = p.vec != 0;
-    // Staging: thread t loads k [8 (t & 1), + 8) of row t >> 1 of both operands.
-    const int row = tid >> 1, kh = (tid & 1) * 8;
-    const float* arow = p.A + (int64_t)min(m0 + row, p.M - 1) * p.lda;
-    const float* brow = p.B + (int64_t)min(n0 + row, p.N - 1) * p.ldb;
+    // Staging: k [4 q, + 4) of two rows of both operands per thread, so four
+    // consecutive lanes load (and write) one row's 64 (32) consecutive bytes.
+    const int row = tid >> 2, kq = (tid & 3) * 4;
+    // VEC: buffer loads, the tile's first row the scalar base, a row's 32-bit
+    // byte offset per lane (f32_validate bounds it), the chunk a scalar offset.
+    const float* grow[4];  // A rows, B rows
+    uint32_t gofs[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int ar = min(row + 64 * i, p.M - 1 - m0), br = min(row + 64 * i, p.N - 1 - n0);
+        if constexpr (VEC) {
+            gofs[i] = (uint32_t)(ar * (int)p.lda + kq) * 4u;
+            gofs[2 + i] = (uint32_t)(br * (int)p.ldb + kq) * 4u;
+        } else {
+            grow[i] = p.A + (m0 + ar) * p.lda + kq;
+            grow[2 + i] = p.B + (n0 + br) * p.ldb + kq;
+        }
+    }
+    const __amdgpu_buffer_rsrc_t rsa =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A + m0 * p.lda), 0, 0x7FFFFFFF, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsb =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B + n0 * p.ldb), 0, 0x7FFFFFFF, 0x00020000);
 
-    constexpr int NSET = 2, FLUSH = 8;  // running sets; chunks per block sum
-    f32x16_t acc[NSET][FN][FM], tot[FN][FM];
+    f32x16_t acc[2][2], low[2][2], tot[2][2];
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                tot[j][i][e] = 0.f;
+            for (int e = 0; e < 16; ++e) acc[j][i][e] = low[j][i][e] = tot[j][i][e] = 0.f;
+
+    float big = 0.f;  // largest |operand| this thread staged
+    const int nk = (p.K + FKC - 1) / FKC, K = p.K;
+    const int wofs = row * 32 + (((kq >> 3) ^ xswz(row)) << 4) + 2 * (kq & 4);
+    float4 raw[4];
+    // Chunks past the last are staged again from it and never read.
+    auto fetch = [&](int kt) {
+        const int k0 = min(kt, nk - 1) * FKC;
 #pragma unroll
-                for (int c = 0; c < NSET; ++c) acc[c][j][i][e] = 0.f;
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (VEC) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(i < 2 ? rsa : rsb, gofs[i], k0 * 4, 0);
+                raw[i] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
+                                     __uint_as_float(v[3]));
+            } else {
+                raw[i] = load4<false>(grow[i], k0, K - kq);
             }
-
-    float4 ra0, ra1, rb0, rb1;
-    auto fetch = [&](int k0) {
-        load8(arow, k0 + kh, p.K, vec, ra0, ra1);
-        load8(brow, k0 + kh, p.K, vec, rb0, rb1);
+        }
     };
-    auto stash = [&](int s) {
-        float* a = &sa[s][row * FKP + kh];
-        float* b = &sb[s][row * FKP + kh];
-        *reinterpret_cast<float4*>(a) = ra0;
-        *reinterpret_cast<float4*>(a + 4) = ra1;
-        *reinterpret_cast<float4*>(b) = rb0;
-        *reinterpret_cast<float4*>(b + 4) = rb1;
+    auto stash = [&](uint8_t* st) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 x = raw[i];
+            uint2 pl[3];
+            split3(x, pl);
+            big = max3_abs(max3_abs(big, x.x, x.y), x.z, x.w);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                *reinterpret_cast<uint2*>(st + wofs + 64 * 32 * i + XPLANE * j) = pl[j];
+        }
     };
 
-    const int lrow = lane & 31, lk = (lane >> 5) * 8;
-    const int nk = (p.K + FKC - 1) / FKC;
+    const int lrow = lane & 31, g = lane >> 5;
+    const int rofs = lrow * 32 + ((g ^ xswz(lrow)) << 4);
+    const int xofs = wm * 32 + rofs, yofs = (FT + wn) * 32 + rofs;
+    typedef bf16x8_t frag2[2];
+    auto read = [&](const uint8_t* st, int ofs, int plane, frag2& f) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            f[j] = *reinterpret_cast<const bf16x8_t*>(st + ofs + XPLANE * plane + 32 * 32 * j);
+    };
+    auto mac = [&](f32x16_t (&c)[2][2], const frag2& wf, const frag2& xf) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                c[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], xf[i], c[j][i], 0, 0, 0);
+    };
     fetch(0);
-    stash(0);
+    stash(smem);
+    fetch(1);
+    stash(smem + XSTAGE);
+    fetch(2);
     __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-        const int s = kt & 1;
-        const bool more = kt + 1 < nk;
-        if (more) fetch((kt + 1) * FKC);
-        float4 w[FN][2], x[FM][2];
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const float* r = &sb[s][(wn + 32 * j + lrow) * FKP + lk];
-            w[j][0] = *reinterpret_cast<const float4*>(r);
-            w[j][1] = *reinterpret_cast<const float4*>(r + 4);
+    uint8_t *s0 = smem, *s1 = smem + XSTAGE, *s2 = smem + 2 * XSTAGE;  // chunk kt, kt + 1, kt + 2
+    for (int kt = 0; kt < nk;) {
+        const int end = min(kt + FLUSH, nk);
+        for (; kt < end; ++kt) {
+            frag2 w0, w1, w2, x0, x1, x2;
+            read(s0, yofs, 0, w0);
+            read(s0, xofs, 0, x0);
+            read(s0, xofs, 1, x1);
+            __builtin_amdgcn_s_setprio(1);
+            mac(acc, w0, x0);
+            read(s0, yofs, 1, w1);
+            mac(low, w0, x1);
+            read(s0, xofs, 2, x2);
+            mac(low, w1, x1);
+            mac(low, w1, x0);
+            read(s0, yofs, 2, w2);
+            mac(low, w0, x2);
+            mac(low, w2, x0);
+            __builtin_amdgcn_s_setprio(0);
+            stash(s2);
+            fetch(kt + 3);
+            // Chunk kt + 2 is written, and every wave has read chunk kt's planes
+            // (chunk kt + 3 takes its stage next).
+            __syncthreads();
+            uint8_t* t = s0;
+            s0 = s1;
+            s1 = s2;
+            s2 = t;
         }
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const float* r = &sa[s][(wm + 32 * i + lrow) * FKP + lk];
-            x[i][0] = *reinterpret_cast<const float4*>(r);
-            x[i][1] = *reinterpret_cast<const float4*>(r + 4);
-        }
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int st = 0; st < 8; ++st) {
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const float wv = w[j][st >> 2][st & 3];
-#pragma unroll
-                for (int i = 0; i < FM; ++i)
-                    acc[st % NSET][j][i] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(wv, x[i][st >> 2][st & 3], acc[st % NSET][j][i], 0, 0, 0);
-            }
-        }
-        if ((kt + 1) % FLUSH == 0 || !more) {
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int i = 0; i < FM; ++i)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        tot[j][i][e] += acc[0][j][i][e] + acc[1][j][i][e];
-                        acc[0][j][i][e] = 0.f;
-                        acc[1][j][i][e] = 0.f;
-                    }
-        }
-        if (more) stash(s ^ 1);
-        __syncthreads();
+                for (int e = 0; e < 16; ++e) {
+                    tot[j][i][e] += acc[j][i][e];
+                    acc[j][i][e] = 0.f;
+                }
     }
 
+    // The split products stand in for fp32 ones only where every part of
+    // them is a normal number: no operand above 2^30 (or not finite), and no
+    // sum small enough for a part that fell below bf16's range to show.  A
+    // sum of operands that are all zero or at least 2^-35 is exact however
+    // small, so a small sum first looks for smaller operands.
+    bool odd = !(big < kSplitMax), small = false;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float v = tot[j][i][e] += low[j][i][e];
+                odd |= !(fabsf(v) < INFINITY);
+                small |= fabsf(v) < kSplitMin;
+            }
+    if (__syncthreads_or(small)) {
+        for (int kt = 0; kt < nk; ++kt) {
+            fetch(kt);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float x[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) odd |= x[e] != 0.f && fabsf(x[e]) < kTiny;
+            }
+        }
+    }
+    if (__syncthreads_or(odd)) f32_tile_native<VEC>(p, smem, m0, n0, wm, wn, tot);
+
     // Epilogue: bias, addend, store 4 consecutive n per lane where they fit.
-    const int g = lane >> 5;
     const bool v4 = (p.N % 4) == 0;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
+    for (int i = 0; i < 2; ++i) {
         const int m = m0 + wm + 32 * i + lrow;
         if (m >= p.M) continue;
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
+        for (int j = 0; j < 2; ++j) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int n = n0 + wn + 32 * j + 8 * q + 4 * g;
@@ -231,9 +413,17 @@ int f32_launch(const F32Problem* ps, int n, hipStream_t st) {
     DT_REQUIRE(total < (1ll << 31), "dt_gemm_f32: too many tiles");
     g.tile_start[n] = (int)total;
     if (total == 0) return DT_OK;
-    hipLaunchKernelGGL(gemm_f32_kernel, dim3((unsigned)total), dim3(256), 0, st, g);
+    bool vec = true;
+    for (int i = 0; i < n; ++i) vec = vec && ps[i].vec;
+    if (vec)
+        hipLaunchKernelGGL(gemm_f32_kernel<true>, dim3((unsigned)total), dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL(gemm_f32_kernel<false>, dim3((unsigned)total), dim3(256), 0, st, g);
     return check_launch("dt_gemm_f32");
 }
+
+// 128 rows of it span less than 2^31 bytes.
+constexpr int64_t kVecLd = (1ll << 22) - 1;
 
 int f32_validate(const dt_gemm_problem& q, F32Problem* out) {
     DT_REQUIRE(q.M >= 0 && q.N >= 0 && q.K > 0, "dt_gemm_f32: bad shape");
@@ -248,7 +438,7 @@ int f32_validate(const dt_gemm_problem& q, F32Problem* out) {
                    "dt_gemm_f32: A and B must be 4-byte aligned");
         DT_REQUIRE(q.N % 4 != 0 || ((reinterpret_cast<uintptr_t>(q.C) & 15) == 0 && q.ldc % 4 == 0),
                    "dt_gemm_f32: C must be 16-byte aligned with ldc %% 4 == 0");
-        vec = q.K % FKC == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && aligned16(q.A) && aligned16(q.B);
+        vec = q.K % FKC == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && q.lda <= kVecLd && q.ldb <= kVecLd && aligned16(q.A) && aligned16(q.B);
     }
     *out = F32Problem{(const float*)q.A, (const float*)q.B, (float*)q.C, (const float*)q.addend, q.bias,
                       q.lda, q.ldb, q.ldc, q.ldd, (int)q.M, (int)q.N, (int)q.K, vec};

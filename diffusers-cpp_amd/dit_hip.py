@@ -646,7 +646,7 @@ def flash_attn(q, k, v, scale=None, out=None, out_dtype=None):
 
 
 def gemm_f32(a, b, bias=None, addend=None, out=None):
-    """a: fp32 [M, K], b: fp32 [N, K] (rows K-contiguous) -> a @ b.T (+ bias) (+ addend), fp32 MFMA."""
+    """a: fp32 [M, K], b: fp32 [N, K] (rows K-contiguous) -> a @ b.T (+ bias) (+ addend), to fp32 accuracy."""
     torch = _torch()
     M, K = a.shape
     N = b.shape[0]

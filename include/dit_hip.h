@@ -420,8 +420,9 @@ int dt_flash_attn_qk_bf16(const void *q0, const int64_t *q0_strides, const float
 /* fp32 counterparts for graphs whose weights and activations are both F32
  * (the reference's own precision: Linear::forward with F32 weights,
  * src/nn/Linear.cpp:17-36, and FlashAttentionOp::operator() on F32 q/k/v,
- * src/nn/attention/FlashAttentionOp.cpp:84-94).  Products and sums in fp32
- * on the fp32 matrix cores.
+ * src/nn/attention/FlashAttentionOp.cpp:84-94).  Products to fp32 accuracy
+ * (operands split exactly into bf16 parts, or fp32 matrix cores where a part
+ * would leave bf16's range), sums in fp32.
  * dt_gemm_f32: C = A B^T (+ bias) (+ addend) as dt_gemm_bf16 with fp32 A
  * [M, K], B [N, K], C and addend (any K; A, B 4-byte aligned; with N % 4 == 0
  * C 16-byte aligned and ldc % 4 == 0).  dt_gemm_f32_grouped: up to 8 of them

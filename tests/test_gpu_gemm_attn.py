@@ -297,7 +297,7 @@ ATTN_SHAPES = [(1, 300, 300, 3), (2, 128, 64, 2), (1, 77, 500, 1), (1, 64, 1, 2)
                                    (129, 260, 12288)])
 def test_gemm_f32(orc, dev, M, N, K):
     """F32 weights with F32 activations (the reference's own Linear precision)
-    on the fp32 matrix cores, against the oracle's linear at the fp32 bar
+    in exact bf16 parts, against the oracle's linear at the fp32 bar
     (|d| <= 1e-5 max(|ref|, 1)); with a bias and an addend; K of any size
     (3 and 40 take the masked loads)."""
     print(f"gemm_f32 M={M} N={N} K={K}", flush=True)
@@ -309,6 +309,55 @@ def test_gemm_f32(orc, dev, M, N, K):
                          bias=dev_tensor(bias, torch.float32), addend=dev_tensor(add, torch.float32))
     torch.cuda.synchronize()
     assert_fp32(host(y), orc.linear(a, b, bias) + add, what=f"gemm_f32 {M}x{N}x{K}")
+
+
+def _f32_edges(case, M, N, K):
+    """Operands around the range in which the fp32 GEMM takes its products in
+    bf16 parts: (a, b), the changed rows or columns inside one 128 x 128 tile."""
+    rng = np.random.default_rng(SEED + 284)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = (0.02 * rng.standard_normal((N, K))).astype(np.float32)
+    if case == "inf":
+        a[5, 3], a[140, 7], b[9, 3] = np.inf, -np.inf, 0.0
+    elif case == "nan":
+        a[130, K - 1], b[2, 0] = np.nan, np.nan
+    elif case == "huge":  # rounds past the largest bf16, and sums near 3e38
+        a[7, :], a[7, 2], b[:, 2] = 0.0, 3.4e38, 0.5
+        a[150] *= np.float32(2.0 ** 60)
+    elif case == "tiny":  # parts and products below the smallest normal number
+        a[3] *= np.float32(2.0 ** -100)
+        b[70] *= np.float32(2.0 ** -110)
+        a[140] *= np.float32(2.0 ** -60)
+    elif case == "zero":
+        a[:, :] = 0.0
+        a[129] = 1.0
+    elif case == "mixed":  # one large element times a tiny one
+        a[4, :], b[8, :] = 0.0, 0.0
+        a[4, 1], b[:, 1] = 2.0 ** 29, 2.0 ** -90
+    return a, b
+
+
+@pytest.mark.parametrize("case", ["inf", "nan", "huge", "tiny", "zero", "mixed"])
+@pytest.mark.parametrize("M,N,K", [(160, 100, 96), (155, 130, 37)])
+def test_gemm_f32_operand_range(dev, case, M, N, K):
+    """Infinities, NaN, the largest and smallest magnitudes, all-zero rows:
+    against 64 bits within K fp32 roundings of the sum of magnitudes (plus one
+    smallest normal number per product), non-finite results the same."""
+    print(f"gemm_f32 {case} {M}x{N}x{K}", flush=True)
+    a, b = _f32_edges(case, M, N, K)
+    y = dit_hip.gemm_f32(dev_tensor(a, torch.float32), dev_tensor(b, torch.float32))
+    torch.cuda.synchronize()
+    got = host(y).astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64).T
+        mag = np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64)).T
+        want = ref.astype(np.float32).astype(np.float64)
+        bad = ~np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), "NaN elsewhere"
+        assert np.array_equal(got[bad & ~np.isnan(want)], want[bad & ~np.isnan(want)]), "infinities differ"
+        ok = ~bad
+        bound = K * (2.0 ** -24 * mag[ok] + 2.0 ** -126)
+        assert (np.abs(got[ok] - ref[ok]) <= bound).all(), np.max(np.abs(got[ok] - ref[ok]) / bound)
 
 
 def test_gemm_f32_strided_in_place(orc, dev):
