@@ -41,6 +41,7 @@
 
 #include "capi_util.hpp"
 #include "common.hpp"
+#include "kernels.hpp"
 
 namespace dit {
 namespace {
@@ -262,6 +263,13 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(const Group grp) {
 // 12-21% faster on every product of the step (4608 x 27648 x 3072: 865 ->
 // 713 us, 1.10 PFLOP/s; 4096 x 4096 x 24576: 1.11 -> 1.24 PFLOP/s), and
 // 14-18% with Q8_0 weights staged.
+// BM = BN = 128 in KG = 2 groups of four waves (64 x 64 each): for products of at most
+// one 128 x 128 tile per CU, where gemm_128_kernel's one k-tile in flight bounds it.
+// Each group multiplies every second k-tile from stages of its own, so twice
+// the DMA is in flight and each SIMD has two waves; the groups' sums are added
+// through LDS at the end.  512 x 3072 x 9216: 105 -> 79 us (bf16), 135 -> 99 us (Q8_0);
+// 1024 x 3072 x 3072: 42 -> 34 us; over more than one tile per CU two
+// workgroups of gemm_128_kernel per CU stay better (512 x 9216 x 3072: 56 against 65 us).
 // BM = 224 (7 blocks of 32): the four waves side by side along n, each
 // 224 x 64 (7 x 2 blocks, 224 accumulators, 9 operand reads for 14 MFMAs).
 // M = 4608 then makes 21 tile rows, so a 4608 x 3072 product is 252 tiles on
@@ -293,26 +301,30 @@ __device__ __forceinline__ int swz8(int r) { return (r ^ (r >> 3)) & 7; }
 // dt_dequant followed by the bf16 GEMM bit for bit.  Each code is converted
 // once per workgroup (the eight-wave gemm_q8_kernel converts each twice, after
 // the LDS read); measured 4-16% faster than it on the step's products.
-template <typename TC, bool SCHED, int BM, bool Q8 = false, int NW = 4>
-__global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
-    static_assert(BM == 256 || BM == 224, "tile height");
+template <typename TC, bool SCHED, int BM, bool Q8 = false, int NW = 4, int BN = 256, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG) void gemm_k64_kernel(const Group grp) {
+    static_assert(BN == 128 || BM == 256 || BM == 224, "tile height");
     static_assert(NW == 4 || (NW == 8 && BM == 256), "eight waves: 256-row tiles");
-    constexpr int WAVES_M = BM == 256 ? 2 : 1, WAVES_N = NW / WAVES_M;
-    constexpr int FM = BM / WAVES_M / 32, FN = 256 / WAVES_N / 32;
-    constexpr int AOPB = BM * EROWB, STAGEB = AOPB + 256 * EROWB, NS = 2;
+    static_assert((BN == 256 && KG == 1) || (BM == 128 && BN == 128 && NW == 4), "K groups: 128 x 128 tiles");
+    constexpr int WAVES_M = BM == 224 ? 1 : 2, WAVES_N = NW / WAVES_M;
+    constexpr int FM = BM / WAVES_M / 32, FN = BN / WAVES_N / 32;
+    constexpr int AOPB = BM * EROWB, STAGEB = AOPB + BN * EROWB, NS = 2;
     constexpr int A_DMA = BM / NW / 8;  // A rows per wave / 8 rows per DMA instruction
-    constexpr int B_DMA = 256 / NW / 8;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[NS * STAGEB];
+    constexpr int B_DMA = BN / NW / 8;
+    __shared__ __attribute__((aligned(16))) uint8_t smem_all[KG * NS * STAGEB];
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    // Group kg of NW waves: k-tiles kg, kg + KG, ... through its own stages.
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW));
+    uint8_t* const smem = smem_all + kg * NS * STAGEB;
+    const int tid = KG == 1 ? threadIdx.x : threadIdx.x % (64 * NW), lane = tid & 63;
     // The wave index is uniform: read it into a scalar so every LDS
     // destination below is a scalar (M0 without a per-instruction
     // readfirstlane).
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tm, tn;
-    const Problem& p = locate<BM, 256>(grp, &tm, &tn);
-    const int m0 = tm * BM, n0 = tn * 256;
-    const int wm = (wave / WAVES_N) * (BM / WAVES_M), wn = (wave % WAVES_N) * (256 / WAVES_N);
+    const Problem& p = locate<BM, BN>(grp, &tm, &tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int wm = (wave / WAVES_N) * (BM / WAVES_M), wn = (wave % WAVES_N) * (BN / WAVES_N);
 
     // DMA sources: wave w fills A rows [BM/NW w, +BM/NW) and B rows
     // [256/NW w, +256/NW), instructions of 8 rows each; lane i covers row +
@@ -329,7 +341,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
     // Q8: thread t stages codes [16 (t % 4), +16) of B rows t / 4 + 16 NW j
     // (j < 16 / NW) and their block scales; they are converted to bf16 and
     // written to the stage one k-tile later (qwrite).
-    constexpr int QJ = 16 / NW, QROWS = 16 * NW;  // weight rows per thread; rows per pass
+    constexpr int QJ = BN / 16 / NW, QROWS = 16 * NW;  // weight rows per thread; rows per pass
     const int qr = tid >> 2, qc = tid & 3;
     uint32_t oq[QJ];
     const float* qs[QJ];
@@ -349,7 +361,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
     }
 #pragma unroll
     for (int j = 0; j < B_DMA; ++j) {
-        const int row = (256 / NW) * wave + 8 * j + (lane >> 3);
+        const int row = (BN / NW) * wave + 8 * j + (lane >> 3);
         const int c = (lane & 7) ^ swz8(row);
         ob[j] = (uint32_t)(((int64_t)(min(n0 + row, p.N - 1) - n0) * p.ldb + c * 8) * 2);
     }
@@ -388,7 +400,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
     };
     auto issue = [&](int kt, int s) {
         uint8_t* abase = smem + s * STAGEB + (BM / NW) * wave * EROWB;
-        uint8_t* bbase = smem + s * STAGEB + AOPB + (256 / NW) * wave * EROWB;
+        uint8_t* bbase = smem + s * STAGEB + AOPB + (BN / NW) * wave * EROWB;
         const int koff = kt * EBK * 2;
         if constexpr (Q8) qload(kt);  // before the A DMA: waiting for the codes leaves the DMA in flight
 #pragma unroll
@@ -445,14 +457,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, FN * FM - (FN + FM), 0);
+            if constexpr (FN * FM > FN + FM) __builtin_amdgcn_sched_group_barrier(0x008, FN * FM - (FN + FM), 0);
         }
     };
 
-    const int nk = p.K / EBK;
-    issue(0, 0);
+    // With K groups every group runs the same number of k-tiles (the barriers
+    // are the workgroup's): one past the last is loaded from it and not
+    // multiplied.
+    const int nkt = p.K / EBK, nk = (nkt + KG - 1) / KG;
+    const auto ktile = [&](int it) { return KG == 1 ? it : min(it * KG + kg, nkt - 1); };
+    issue(ktile(0), 0);
     if constexpr (Q8) qwrite(0);
-    if (nk > 1) issue(1, 1);
+    if (nk > 1) issue(ktile(1), 1);
     if (nk > 1) wait_vm<A_DMA + B_DMA>();  // Q8: QJ code and QJ scale loads stand in for the B_DMA B DMAs
     else wait_vm<0>();
     if constexpr (Q8) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the B rows written
@@ -480,7 +496,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
         wait_vm<0>();
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
-        if constexpr (decltype(issue_next)::value) issue(kt + 2, s);
+        if constexpr (decltype(issue_next)::value) issue(ktile(kt + 2), s);
         read_ops(s ^ 1, 0, wa, xa);
         mfma(wb, xb);
         if constexpr (SCHED) {
@@ -495,7 +511,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
     };
     for (int kt = 0; kt < nk - 2; ++kt) body(kt, std::true_type{});
     if (nk >= 2) body(nk - 2, std::false_type{});
-    {
+    if (KG == 1 || (nk - 1) * KG + kg < nkt) {
         const int s = (nk - 1) & 1;
         read_ops(s, 1, wb, xb);
         mfma(wa, xa);
@@ -507,6 +523,33 @@ __global__ __launch_bounds__(64 * NW) void gemm_k64_kernel(const Group grp) {
         mfma(wa, xa);
         pipe();
         mfma(wb, xb);
+    }
+    if constexpr (KG > 1) {
+        // The groups' sums meet in LDS (all stages have been read) and are
+        // added in group order by the first.
+        float* part = reinterpret_cast<float*>(smem_all);
+        constexpr int PW = FM * FN * 16 * 64;
+        __syncthreads();
+        if (kg > 0) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        part[((kg - 1) * NW + wave) * PW + ((j * FM + i) * 16 + e) * 64 + lane] = acc[j][i][e];
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        acc[j][i][e] += part[(q * NW + wave) * PW + ((j * FM + i) * 16 + e) * 64 + lane];
     }
     epilogue<FM, FN, TC>(p, acc, m0 + wm, n0 + wn, lane);
 }
@@ -852,6 +895,107 @@ __global__ __launch_bounds__(256) void gemm_128_kernel(const Group grp) {
     epilogue<FM, FN, TC>(p, acc, m0 + wm, n0 + wn, lane);
 }
 
+// ---- few rows: 16 weight rows per workgroup, K split over its waves -------------
+// M <= 16 (a conditioning vector's Linear): the product is a stream of the
+// weight.  With 128 x 128 tiles its 18432 x 3072 (113 MB) took 40.8 us at M = 1 with
+// 576 waves, each holding one k-tile in flight behind a barrier; here 27.4 us
+// (4.1 TB/s), 3072 x 9216 101 -> 19 us.
+// Every wave reads its weights straight into the MFMA's operand registers,
+// without LDS or barriers: a workgroup owns 16 weight rows, its KS waves one K
+// range each, and a wave loads four blocks of 64 k (16 rows x 128 bytes, whole
+// lines) at once; the partial sums meet in LDS and are added in wave order.
+// The activations (L2-resident) are read the same way by every workgroup.
+// v_mfma_f32_16x16x32_bf16 with the weights as A: lane l supplies row l % 16,
+// k = 64 b + 16 (l / 16) + 8 s + [0, 8) in step s of block b -- for both
+// operands, so the sum only meets its terms in another order -- and holds
+// C[m = l % 16][n = 4 (l / 16) + i].
+// Q8: 16 codes of one row per lane and block, w = fma(u, d, -128 d) rounded to
+// bf16, the value dt_dequant writes.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+template <typename TC, bool Q8, int KS>
+__global__ __launch_bounds__(64 * KS) void gemm_skinny_kernel(const Group grp) {
+    constexpr int UNR = 4;      // 64-k blocks loaded together
+    constexpr int LD = 16 + 4;  // padded row of the partial sums
+    __shared__ float part[KS][16 * LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int pi = 0;
+    while (pi + 1 < grp.count && (int)blockIdx.x >= grp.tile_start[pi + 1]) ++pi;
+    const Problem& p = grp.p[pi];
+    const int n0 = ((int)blockIdx.x - grp.tile_start[pi]) * 16;
+    const int r = lane & 15, g = lane >> 4;
+
+    const int nblk = p.K / 64, per = (nblk + KS - 1) / KS;
+    const int b0 = min(wave * per, nblk), b1 = min(b0 + per, nblk);
+    const uint16_t* xp = p.A + (int64_t)min(r, p.M - 1) * p.lda + 16 * g;
+    const int64_t n = min(n0 + r, p.N - 1);
+    const uint16_t* wp = Q8 ? nullptr : p.B + n * p.ldb + 16 * g;
+    const uint8_t* qp = Q8 ? reinterpret_cast<const uint8_t*>(p.B) + n * p.ldb + 16 * g : nullptr;
+    const float* sp = Q8 ? p.Bs + n + (g >> 1) * p.ldbs : nullptr;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+
+    // U blocks from block b.
+    auto step = [&](int b, auto uc) {
+        constexpr int U = decltype(uc)::value;
+        uint4 w[U][2], x[U][2];
+        float d[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = (int64_t)(b + u) * 64;
+            if constexpr (Q8) {
+                w[u][0] = ld_stream(qp + k);
+                d[u] = sp[2 * (int64_t)(b + u) * p.ldbs];
+            } else {
+                w[u][0] = ld_stream(wp + k);
+                w[u][1] = ld_stream(wp + k + 8);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[u][h] = *reinterpret_cast<const uint4*>(xp + k + 8 * h);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if constexpr (Q8) {
+                const float m = -128.0f * d[u];
+                const uint32_t q4[4] = {w[u][0].x, w[u][0].y, w[u][0].z, w[u][0].w};
+                uint32_t pk[8];
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf((float)((q4[h] >> (8 * e)) & 0xFFu), d[u], m);
+                    pk[2 * h] = pack_bf16x2(v[0], v[1]);
+                    pk[2 * h + 1] = pack_bf16x2(v[2], v[3]);
+                }
+                w[u][0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+                w[u][1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[u][h]),
+                                                              __builtin_bit_cast(bf16x8_t, x[u][h]), acc, 0, 0, 0);
+        }
+    };
+    int b = b0;
+    for (; b + UNR <= b1; b += UNR) step(b, std::integral_constant<int, UNR>{});
+    for (; b < b1; ++b) step(b, std::integral_constant<int, 1>{});
+
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[wave][r * LD + 4 * g + e] = acc[e];
+    __syncthreads();
+    TC* C = reinterpret_cast<TC*>(p.C);
+    const TC* Dm = reinterpret_cast<const TC*>(p.D);
+    for (int u = tid; u < 16 * 16; u += 64 * KS) {
+        const int m = u >> 4, c = u & 15;
+        if (m >= p.M || n0 + c >= p.N) continue;
+        float v = part[0][m * LD + c];
+#pragma unroll
+        for (int k = 1; k < KS; ++k) v += part[k][m * LD + c];
+        if (p.bias) v += p.bias[n0 + c];
+        if (Dm) v += load_c(Dm + (int64_t)m * p.ldd + n0 + c);
+        store1<TC>(C + (int64_t)m * p.ldc + n0 + c, v);
+    }
+}
+
 // ---- any shape: 128 x 128, K in steps of 16 under a bounds mask ---------------
 // For the GEMMs the kernels above do not take: K not a multiple of 64 (ggml's
 // mul_mat takes any K, e.g. a ResnetBlock2D's time-embedding projection with
@@ -943,11 +1087,25 @@ struct Config {
 // 5: config 2 with the operand reads interleaved into the MFMA stream; 6: the
 // same at 224 x 256; 7: config 5 with Q8_0 weights dequantised as they are
 // staged; 8, 9: configs 5 and 7 in eight waves of 128 x 64 (two per SIMD).
+// Chosen by size only, not by callers: 10: few rows (gemm_skinny_kernel); 11: 128 x 128
+// in two k-groups (the rate puts it below config 1's pair of tiles per CU only
+// while one round of it holds every tile).
 constexpr int kAnyConfig = 4, kLastConfig = 9;
-constexpr Config kConfigs[10] = {{256, 256, 512, 1, 1.15}, {128, 128, 256, 2, 0.9}, {256, 256, 256, 1, 1.15},
+constexpr int kSkinnyConfig = 10, kSplitConfig = 11;
+// Rows up to which the weight stream wins (Python call included, bf16 / Q8_0; the
+// tiles, K split where it is): 18432 x 3072 at 16 rows 37.9 / 27.5 us against 40.7 /
+// 46.3, at 32 rows 48.1 / 35.6 against 29.3 / 36.4, its activations being read
+// again for every 16 weight rows.
+constexpr int kSkinnyM = 16;
+// Weights of fewer elements keep one running sum over ascending k, the order of
+// every configuration a caller can name (C is then the same bits in all of
+// them); a larger weight's few-tile product sums K ranges.
+constexpr int64_t kRangeWeight = 1 << 20;
+bool sums_ranges(int64_t N, int64_t K) { return N * K >= kRangeWeight; }
+constexpr Config kConfigs[12] = {{256, 256, 512, 1, 1.15}, {128, 128, 256, 2, 0.9}, {256, 256, 256, 1, 1.15},
                                 {256, 256, 512, 1, 1.0},  {128, 128, 256, 2, 0.1}, {256, 256, 256, 1, 1.3},
                                 {224, 256, 256, 1, 1.2},  {256, 256, 256, 1, 1.25}, {256, 256, 512, 1, 1.3},
-                                {256, 256, 512, 1, 1.3}};
+                                {256, 256, 512, 1, 1.3},  {16, 16, 256, 1, 0.1},  {128, 128, 512, 1, 0.6}};
 
 int64_t tiles_of(const Problem& p, int cfg) {
     const Config c = kConfigs[cfg];
@@ -984,17 +1142,43 @@ int pick_by_waves(const Problem* ps, int n, int cus, std::initializer_list<int> 
 // CUs idle (the 512 text tokens' 3072-column products, a 128-column output),
 // 128 x 128 tiles dequantised the same way (512 x 3072 x 9216: 135 against
 // 203 us).
-int pick_config_q8(const Problem* ps, int n, int cus) { return pick_by_waves(ps, n, cus, {9, 1}); }
+int pick_config_q8(const Problem* ps, int n, int cus, bool ranges) {
+    return ranges ? pick_by_waves(ps, n, cus, {9, 1, kSplitConfig}) : pick_by_waves(ps, n, cus, {9, 1});
+}
 
 // bf16 weights: the eight-wave K = 64 kernel's 256 x 256 tiles (config 8), or
 // 128 x 128 tiles for the products with few tiles.  Config 8 measured faster
 // than the four-wave 224 x 256 tiles on every product of the step that those
 // took (4608 x 3072 x 9216: 210 against 225 us; 4608 x 3072 x 3072: 81.5
 // against 91.6 us), so they are no longer a candidate.
-int pick_config(const Problem* ps, int n, int cus) { return pick_by_waves(ps, n, cus, {8, 1}); }
+int pick_config(const Problem* ps, int n, int cus, bool ranges) {
+    return ranges ? pick_by_waves(ps, n, cus, {8, 1, kSplitConfig}) : pick_by_waves(ps, n, cus, {8, 1});
+}
+
+template <typename TC, bool Q8>
+int launch_skinny(const Problem* ps, int n, hipStream_t st) {
+    Group g{};
+    g.count = n;
+    int64_t total = 0;
+    for (int i = 0; i < n; ++i) {
+        g.p[i] = ps[i];
+        g.tile_start[i] = (int)total;
+        total += ((int64_t)ps[i].N + 15) / 16;
+    }
+    DT_REQUIRE(total < (1ll << 31), "dt_gemm_bf16: too many tiles");
+    g.tile_start[n] = (int)total;
+    // Eight waves a workgroup until there are four workgroups per CU.
+    if (total >= 4 * cu_count())
+        hipLaunchKernelGGL((gemm_skinny_kernel<TC, Q8, 4>), dim3((unsigned)total), dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((gemm_skinny_kernel<TC, Q8, 8>), dim3((unsigned)total), dim3(512), 0, st, g);
+    return check_launch("dt_gemm_bf16");
+}
 
 template <typename TC>
 int launch(const Problem* ps, int n, int cfg, hipStream_t st) {
+    if (cfg == kSkinnyConfig)
+        return ps[0].Bs ? launch_skinny<TC, true>(ps, n, st) : launch_skinny<TC, false>(ps, n, st);
     Group g{};
     g.count = n;
     int64_t total = 0;
@@ -1023,6 +1207,10 @@ int launch(const Problem* ps, int n, int cfg, hipStream_t st) {
         hipLaunchKernelGGL((gemm_k64_kernel<TC, true, 256, true, 8>), grid, block, 0, st, g);
     else if (cfg == 3)
         hipLaunchKernelGGL((gemm_q8_kernel<TC>), grid, block, 0, st, g);
+    else if (cfg == kSplitConfig && ps[0].Bs)
+        hipLaunchKernelGGL((gemm_k64_kernel<TC, true, 128, true, 4, 128, 2>), grid, block, 0, st, g);
+    else if (cfg == kSplitConfig)
+        hipLaunchKernelGGL((gemm_k64_kernel<TC, true, 128, false, 4, 128, 2>), grid, block, 0, st, g);
     else if (cfg == kAnyConfig && ps[0].Bs)
         hipLaunchKernelGGL((gemm_any_kernel<TC, true>), grid, block, 0, st, g);
     else if (cfg == kAnyConfig)
@@ -1065,6 +1253,77 @@ int validate(const dt_gemm_problem& q, int32_t c_type, Problem* out, bool* tiled
     return DT_OK;
 }
 
+// ---- one product over K ranges -----------------------------------------------
+// C = sum over s of part[s] (+ bias) (+ addend), part [S][M][ldp] fp32.
+template <typename TC>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int S, int64_t stride,
+                                                          int64_t ldp, TC* C, int64_t ldc, const float* bias,
+                                                          const TC* D, int64_t ldd, int M, int N) {
+    const int n = (blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
+    if (n >= N) return;
+    const float* p = part + (int64_t)m * ldp + n;
+    float4 v = *reinterpret_cast<const float4*>(p);
+    for (int s = 1; s < S; ++s) {
+        const float4 w = *reinterpret_cast<const float4*>(p + s * stride);
+        v.x += w.x;
+        v.y += w.y;
+        v.z += w.z;
+        v.w += w.w;
+    }
+    float o[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) continue;
+        if (bias) o[e] += bias[n + e];
+        if (D) o[e] += load_c(D + (int64_t)m * ldd + n + e);
+    }
+    TC* dst = C + (int64_t)m * ldc + n;
+    if (N % 4 == 0) {
+        store4<TC>(dst, o);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) store1<TC>(dst + e, o[e]);
+    }
+}
+
+}  // namespace
+
+int gemm_reduce(const float* part, int S, int64_t M, int64_t N, void* C, int64_t ldc, const float* bias,
+                const void* addend, int64_t ldd, int32_t c_type, hipStream_t st) {
+    const int64_t ldp = gemm_split_ld(N), stride = M * ldp;
+    for (int64_t m0 = 0; m0 < M; m0 += 65535) {
+        const int64_t rows = M - m0 < 65535 ? M - m0 : 65535;
+        const dim3 grid((unsigned)((N + 1023) / 1024), (unsigned)rows);
+        if (c_type == DT_TYPE_F32)
+            hipLaunchKernelGGL(gemm_reduce_kernel<float>, grid, dim3(256), 0, st, part + m0 * ldp, S, stride, ldp,
+                               (float*)C + m0 * ldc, ldc, bias, addend ? (const float*)addend + m0 * ldd : nullptr,
+                               ldd, (int)rows, (int)N);
+        else
+            hipLaunchKernelGGL(gemm_reduce_kernel<bf16>, grid, dim3(256), 0, st, part + m0 * ldp, S, stride, ldp,
+                               (bf16*)C + m0 * ldc, ldc, bias, addend ? (const bf16*)addend + m0 * ldd : nullptr,
+                               ldd, (int)rows, (int)N);
+        const int rc = check_launch("dt_gemm(reduce)");
+        if (rc) return rc;
+    }
+    return DT_OK;
+}
+
+namespace {
+// K ranges of one product (1: not split): as many as keep one 128 x 128 tile per
+// CU, each at least 512 k (four rounds of the kernel's two k-groups).  3072 x
+// 9216 with the Python call around it (bf16): 128 rows, 24 tiles, 77 us in one range and 27
+// in eight; 512 rows 79 and 53 (two); 768 rows 79 and 76 in three, more than one
+// tile per CU, where 512 rows in five took 62: past one round the tiles share
+// the L2's bandwidth and the partial sums cost what is won.
+int split_count(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+    if (M <= kSkinnyM || K % 64 != 0 || tiles > cus || !sums_ranges(N, K)) return 1;
+    int64_t s = cus / tiles;
+    if (s > K / 512) s = K / 512;
+    if (s > kMaxGroup) s = kMaxGroup;
+    return s < 2 ? 1 : (int)s;
+}
 }  // namespace
 }  // namespace dit
 
@@ -1097,10 +1356,17 @@ extern "C" int dt_gemm_bf16_grouped(const dt_gemm_problem* problems, int32_t cou
     DT_REQUIRE(config == -1 || config == kAnyConfig || all_tiled,
                "dt_gemm_bf16: config %d needs K %% 64 == 0 and 16-byte aligned rows", config);
     if (n == 0) return DT_OK;
+    int m_max = 0;
+    bool ranges = true;
+    for (int i = 0; i < n; ++i) {
+        m_max = m_max > ps[i].M ? m_max : ps[i].M;
+        ranges = ranges && sums_ranges(ps[i].N, ps[i].K);
+    }
     const int cfg = config >= 0      ? config
                     : !all_tiled     ? kAnyConfig
-                    : n_q8           ? pick_config_q8(ps, n, cu_count())
-                                     : pick_config(ps, n, cu_count());
+                    : ranges && m_max <= kSkinnyM ? kSkinnyConfig
+                    : n_q8           ? pick_config_q8(ps, n, cu_count(), ranges)
+                                     : pick_config(ps, n, cu_count(), ranges);
     hipStream_t st = (hipStream_t)stream;
     return c_type == DT_TYPE_F32 ? launch<float>(ps, n, cfg, st) : launch<bf16>(ps, n, cfg, st);
 }
@@ -1124,4 +1390,46 @@ extern "C" int dt_gemm_bf16(const void* A, int64_t lda, const void* B, int64_t l
                             int64_t M, int64_t N, int64_t K, const float* bias, const void* addend,
                             int64_t ldd, int32_t c_type, dt_stream_t stream) {
     return dt_gemm_bf16_config(A, lda, B, ldb, C, ldc, M, N, K, bias, addend, ldd, c_type, -1, stream);
+}
+
+extern "C" size_t dt_gemm_bf16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    using namespace dit;
+    if (M <= 0 || N <= 0 || K <= 0 || M >= (1ll << 31) || N >= (1ll << 31)) return 0;
+    const int s = split_count(M, N, K, cu_count());
+    return s > 1 ? (size_t)(s * M * gemm_split_ld(N)) * sizeof(float) : 0;
+}
+
+extern "C" int dt_gemm_bf16_ws(const dt_gemm_problem* problem, int32_t c_type, void* workspace, size_t workspace_bytes,
+                               dt_stream_t stream) {
+    using namespace dit;
+    DT_REQUIRE(problem != nullptr, "dt_gemm_bf16_ws: null problem");
+    const dt_gemm_problem& q = *problem;
+    const size_t need = dt_gemm_bf16_workspace_bytes(q.M, q.N, q.K);
+    Problem p;
+    bool tiled = false;
+    if (need == 0 || !workspace || workspace_bytes < need || !aligned16(workspace))
+        return dt_gemm_bf16_grouped(problem, 1, c_type, -1, stream);
+    DT_REQUIRE(is_io_type(c_type), "dt_gemm_bf16_ws: c_type %d unsupported", c_type);
+    const int rc = validate(q, c_type, &p, &tiled);
+    if (rc) return rc;
+    if (!tiled) return dt_gemm_bf16_grouped(problem, 1, c_type, -1, stream);
+    const int S = split_count(q.M, q.N, q.K, cu_count());
+    const int64_t ldp = gemm_split_ld(q.N), blocks = q.K / 64;
+    Problem ps[kMaxGroup];
+    float* part = (float*)workspace;
+    for (int s = 0; s < S; ++s) {
+        const int64_t k0 = blocks * s / S * 64, k1 = blocks * (s + 1) / S * 64;
+        ps[s] = p;
+        ps[s].A = p.A + k0;
+        ps[s].B = p.Bs ? reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(p.B) + k0) : p.B + k0;
+        if (p.Bs) ps[s].Bs = p.Bs + k0 / 32 * p.ldbs;
+        ps[s].K = (int)(k1 - k0);
+        ps[s].C = part + s * q.M * ldp;
+        ps[s].ldc = ldp;
+        ps[s].D = nullptr;
+        ps[s].bias = nullptr;
+    }
+    const int rl = launch<float>(ps, S, kSplitConfig, (hipStream_t)stream);
+    if (rl) return rl;
+    return gemm_reduce(part, S, q.M, q.N, q.C, q.ldc, q.bias, q.addend, q.ldd, c_type, (hipStream_t)stream);
 }

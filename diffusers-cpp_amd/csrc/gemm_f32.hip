@@ -47,8 +47,11 @@
 // taken eight at a time through a workspace -- the fp32 arithmetic of ggml's
 // CPU flash_attn_ext for F32 operands (FlashAttentionOp.cpp:84-94), with the
 // probabilities normalised before the product instead of after.
+#include <type_traits>
+
 #include "capi_util.hpp"
 #include "common.hpp"
+#include "kernels.hpp"
 
 namespace dit {
 namespace {
@@ -399,9 +402,131 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
     }
 }
 
+// ---- few rows -----------------------------------------------------------------
+// The product is a stream of the weight, and the fp32 matrix cores keep up with
+// it (18432 x 3072 at 16 rows: 12 us of v_mfma_f32_16x16x4_f32 against 44 us of
+// weights at 5.1 TB/s), so nothing is split into bf16 parts.  As the bf16
+// kernel for few rows (gemm.hip): a workgroup owns 16 weight rows, its KS waves one K range
+// each, operands go straight from memory into registers, and the partial sums
+// meet in LDS and are added in wave order.  Lane l supplies row l % 16, k = 16 b +
+// 4 (l / 16) + s in MFMA s of 16-k block b.  Each s has a running sum of its own over 8
+// blocks; the four are added and join the wave's total (one running sum was
+// 20% less exact than the tiles, this is more).  At M = 1 18432 x 3072 341 ->
+// 59 us, 3072 x 3072 339 -> 18 us.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// Up to 16 rows; up to 32 with fewer than four workgroups per CU (3072 x 3072 at 20 rows
+// 22.5 us against 38 in tiles; 18432 x 3072 104 against 86, its activations
+// being read again for every 16 weight rows).
+bool f32_skinny(int64_t M, int64_t cols) { return M <= 16 || (M <= 32 && (cols + 15) / 16 < 4 * cu_count()); }
+
+template <int MB, int KS>
+__global__ __launch_bounds__(64 * KS) void gemm_f32_skinny_kernel(const F32Group grp) {
+    constexpr int LD = 16 + 4;
+    __shared__ float part[KS][16 * MB * LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int pi = 0;
+    while (pi + 1 < grp.count && (int)blockIdx.x >= grp.tile_start[pi + 1]) ++pi;
+    const F32Problem& p = grp.p[pi];
+    const int n0 = ((int)blockIdx.x - grp.tile_start[pi]) * 16;
+    const int r = lane & 15, g = lane >> 4;
+    const int nblk = p.K / 16, per = (nblk + KS - 1) / KS;
+    const int b0 = min(wave * per, nblk), b1 = min(b0 + per, nblk);
+    const float* wp = p.B + (int64_t)min(n0 + r, p.N - 1) * p.ldb + 4 * g;
+    const float* xp[MB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) xp[i] = p.A + (int64_t)min(16 * i + r, p.M - 1) * p.lda + 4 * g;
+    f32x4_t tot[MB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    // U blocks from block b: one run.
+    auto run = [&](int b, auto uc) {
+        constexpr int U = decltype(uc)::value;
+        float4 w[U], x[U][MB];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint4 t = ld_stream(wp + (int64_t)(b + u) * 16);
+            w[u] = make_float4(__uint_as_float(t.x), __uint_as_float(t.y), __uint_as_float(t.z), __uint_as_float(t.w));
+#pragma unroll
+            for (int i = 0; i < MB; ++i) x[u][i] = *reinterpret_cast<const float4*>(xp[i] + (int64_t)(b + u) * 16);
+        }
+        f32x4_t acc[MB][4];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc[i][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float wv[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                const float xv[4] = {x[u][i].x, x[u][i].y, x[u][i].z, x[u][i].w};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    acc[i][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s], xv[s], acc[i][s], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tot[i][e] += (acc[i][0][e] + acc[i][1][e]) + (acc[i][2][e] + acc[i][3][e]);
+    };
+    int b = b0;
+    for (; b + 8 <= b1; b += 8) run(b, std::integral_constant<int, 8>{});
+    for (; b + 2 <= b1; b += 2) run(b, std::integral_constant<int, 2>{});
+    if (b < b1) run(b, std::integral_constant<int, 1>{});
+
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[wave][(16 * i + r) * LD + 4 * g + e] = tot[i][e];
+    __syncthreads();
+    for (int u = tid; u < 16 * MB * 16; u += 64 * KS) {
+        const int m = u >> 4, c = u & 15, n = n0 + c;
+        if (m >= p.M || n >= p.N) continue;
+        float v = part[0][m * LD + c];
+#pragma unroll
+        for (int k = 1; k < KS; ++k) v += part[k][m * LD + c];
+        if (p.bias) v += p.bias[n];
+        if (p.D) v += p.D[(int64_t)m * p.ldd + n];
+        p.C[(int64_t)m * p.ldc + n] = v;
+    }
+}
+
+template <int MB>
+int f32_skinny_launch(const F32Problem* ps, int n, hipStream_t st) {
+    F32Group g{};
+    g.count = n;
+    int64_t total = 0;
+    for (int i = 0; i < n; ++i) {
+        g.p[i] = ps[i];
+        g.tile_start[i] = (int)total;
+        total += ((int64_t)ps[i].N + 15) / 16;
+    }
+    DT_REQUIRE(total < (1ll << 31), "dt_gemm_f32: too many tiles");
+    g.tile_start[n] = (int)total;
+    // Eight waves a workgroup until there are four workgroups per CU.
+    if (total >= 4 * cu_count())
+        hipLaunchKernelGGL((gemm_f32_skinny_kernel<MB, 4>), dim3((unsigned)total), dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((gemm_f32_skinny_kernel<MB, 8>), dim3((unsigned)total), dim3(512), 0, st, g);
+    return check_launch("dt_gemm_f32");
+}
+
 int64_t f32_tiles(const F32Problem& p) { return (int64_t)((p.M + FT - 1) / FT) * ((p.N + FT - 1) / FT); }
 
 int f32_launch(const F32Problem* ps, int n, hipStream_t st) {
+    int m_max = 0;
+    int64_t cols = 0;
+    bool vec = true;
+    for (int i = 0; i < n; ++i) {
+        vec = vec && ps[i].vec;
+        m_max = m_max > ps[i].M ? m_max : ps[i].M;
+        cols += ps[i].N;
+    }
+    if (vec && f32_skinny(m_max, cols))
+        return m_max <= 16 ? f32_skinny_launch<1>(ps, n, st) : f32_skinny_launch<2>(ps, n, st);
     F32Group g{};
     g.count = n;
     int64_t total = 0;
@@ -413,8 +538,6 @@ int f32_launch(const F32Problem* ps, int n, hipStream_t st) {
     DT_REQUIRE(total < (1ll << 31), "dt_gemm_f32: too many tiles");
     g.tile_start[n] = (int)total;
     if (total == 0) return DT_OK;
-    bool vec = true;
-    for (int i = 0; i < n; ++i) vec = vec && ps[i].vec;
     if (vec)
         hipLaunchKernelGGL(gemm_f32_kernel<true>, dim3((unsigned)total), dim3(256), 0, st, g);
     else
@@ -514,6 +637,67 @@ extern "C" int dt_gemm_f32(const float* A, int64_t lda, const float* B, int64_t 
                            dt_stream_t stream) {
     const dt_gemm_problem p{A, lda, B, ldb, C, ldc, addend, ldd, bias, M, N, K, nullptr, 0};
     return dt_gemm_f32_grouped(&p, 1, stream);
+}
+
+// K ranges of one product (1: not split), for products of at most two tiles per
+// CU (a CU runs two at once): the number with the least estimated time, rounds
+// of workgroups at 6.3 us per 128 k of one tile alone on its CU and 10.2 beside
+// another (both measured), then the reduce, its launch and the partial sums at
+// 5 TB/s.  A range has at least 512 k.  3072 x 9216, Python call included: 200 rows
+// 456 us in one range, 99 in eight; 1536 rows 647 and 496 (five).
+static int f32_split_count(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + dit::FT - 1) / dit::FT) * ((N + dit::FT - 1) / dit::FT), cus = dit::cu_count();
+    if (dit::f32_skinny(M, N) || K % 64 != 0 || tiles > 2 * cus) return 1;
+    int best = 1;
+    double best_t = 1e300;
+    for (int64_t S = 1; S <= dit::kF32MaxGroup && (S == 1 || S <= K / 512); ++S) {
+        const int64_t full = tiles * S / (2 * cus), rest = tiles * S - full * 2 * cus;
+        const double rounds = (double)full * 10.2 + (rest > cus ? 10.2 : rest > 0 ? 6.3 : 0.0);
+        const double t = rounds * (double)K / (double)(128 * S) +
+                         (S > 1 ? 5.0 + (double)(S * M * N) * 8.0 / 5.0e6 : 0.0);
+        if (t < best_t) {
+            best_t = t;
+            best = (int)S;
+        }
+    }
+    return best;
+}
+
+extern "C" size_t dt_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || M >= (1ll << 31) || N >= (1ll << 31)) return 0;
+    const int s = f32_split_count(M, N, K);
+    return s > 1 ? (size_t)(s * M * dit::gemm_split_ld(N)) * sizeof(float) : 0;
+}
+
+extern "C" int dt_gemm_f32_ws(const dt_gemm_problem* problem, void* workspace, size_t workspace_bytes,
+                              dt_stream_t stream) {
+    using namespace dit;
+    DT_REQUIRE(problem != nullptr, "dt_gemm_f32_ws: null problem");
+    const dt_gemm_problem& q = *problem;
+    const size_t need = dt_gemm_f32_workspace_bytes(q.M, q.N, q.K);
+    if (need == 0 || !workspace || workspace_bytes < need || !aligned16(workspace))
+        return dt_gemm_f32_grouped(problem, 1, stream);
+    F32Problem p;
+    const int rc = f32_validate(q, &p);
+    if (rc) return rc;
+    const int S = f32_split_count(q.M, q.N, q.K);
+    const int64_t ldp = gemm_split_ld(q.N), blocks = q.K / 64;
+    F32Problem ps[kF32MaxGroup];
+    float* part = (float*)workspace;
+    for (int s = 0; s < S; ++s) {
+        const int64_t k0 = blocks * s / S * 64, k1 = blocks * (s + 1) / S * 64;
+        ps[s] = p;
+        ps[s].A = p.A + k0;
+        ps[s].B = p.B + k0;
+        ps[s].K = (int)(k1 - k0);
+        ps[s].C = part + s * q.M * ldp;
+        ps[s].ldc = ldp;
+        ps[s].D = nullptr;
+        ps[s].bias = nullptr;
+    }
+    const int rl = f32_launch(ps, S, (hipStream_t)stream);
+    if (rl) return rl;
+    return gemm_reduce(part, S, q.M, q.N, q.C, q.ldc, q.bias, q.addend, q.ldd, DT_TYPE_F32, (hipStream_t)stream);
 }
 
 // Workspace of dt_flash_attn_f32: per head of a group of up to 8, the

@@ -82,6 +82,12 @@ int gn_tile_stats_finalize(const void* stats, int64_t N, int64_t groups, int64_t
 // (resolved once per device).
 int noalloc_scratch(void** out);
 
+// Partial sums of a product taken over S ranges of K, fp32 [S][M][gemm_split_ld(N)]:
+// C = their sum in range order (+ bias) (+ addend).
+inline int64_t gemm_split_ld(int64_t N) { return (N + 3) / 4 * 4; }
+int gemm_reduce(const float* part, int S, int64_t M, int64_t N, void* C, int64_t ldc, const float* bias,
+                const void* addend, int64_t ldd, int32_t c_type, hipStream_t st);
+
 // Backend accessors (capi.cpp).
 hipStream_t backend_stream(dt_backend* be);
 int backend_device(dt_backend* be);

@@ -122,6 +122,10 @@ _SIGS = {
     "dt_q8_0_split_bytes": (c_int64, [c_int64, c_int64]),
     "dt_gemm_f32": (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                               c_void_p, c_void_p, c_int64, _S]),
+    "dt_gemm_bf16_workspace_bytes": (ctypes.c_size_t, [c_int64, c_int64, c_int64]),
+    "dt_gemm_bf16_ws": (c_int32, [c_void_p, c_int32, c_void_p, ctypes.c_size_t, _S]),
+    "dt_gemm_f32_workspace_bytes": (ctypes.c_size_t, [c_int64, c_int64, c_int64]),
+    "dt_gemm_f32_ws": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, _S]),
     "dt_gemm_f32_grouped": (c_int32, [c_void_p, c_int32, _S]),
     "dt_flash_attn_f32_workspace_bytes": (ctypes.c_size_t, [c_int64, c_int64, c_int64, c_int64, c_int64]),
     "dt_flash_attn_f32": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
@@ -480,6 +484,12 @@ def quantize_q8_0(x, out=None):
     return y
 
 
+def _gemm_ws(nbytes, M, N, K, a):
+    """Scratch for a product taken over ranges of K, or None for one that is not split."""
+    n = nbytes(M, N, K)
+    return _torch().empty(n, dtype=_torch().uint8, device=a.device) if n else None
+
+
 def gemm(a, b, bias=None, addend=None, out=None, out_dtype=None, config=-1):
     """a: bf16 [M, K], b: bf16 [N, K] (rows K-contiguous) -> a @ b.T (+ bias) (+ addend).
     config: tile configuration (0: 256x256, 8 waves, K = 32 stages; 1: 128x128;
@@ -492,6 +502,12 @@ def gemm(a, b, bias=None, addend=None, out=None, out_dtype=None, config=-1):
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype or torch.bfloat16, device=a.device)
     ldd = addend.stride(0) if addend is not None else 0
+    ws = _gemm_ws(load().dt_gemm_bf16_workspace_bytes, M, N, K, a) if config == -1 else None
+    if ws is not None:
+        p = GemmProblem(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), out.data_ptr(), out.stride(0),
+                        _p(addend), ldd, _p(bias), M, N, K, None, 0)
+        check(load().dt_gemm_bf16_ws(ctypes.byref(p), io_type(out), _p(ws), ws.numel(), stream()), "dt_gemm_bf16_ws")
+        return out
     check(load().dt_gemm_bf16_config(_p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0),
                                      M, N, K, _p(bias), _p(addend), ldd, io_type(out), config,
                                      stream()),
@@ -534,6 +550,12 @@ def gemm_q8_0(a, w, bias=None, addend=None, out=None, out_dtype=None):
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype or torch.bfloat16, device=a.device)
     ldd = addend.stride(0) if addend is not None else 0
+    ws = _gemm_ws(load().dt_gemm_bf16_workspace_bytes, M, N, K, a)
+    if ws is not None:
+        p = GemmProblem(a.data_ptr(), a.stride(0), w.codes.data_ptr(), w.codes.stride(0), out.data_ptr(),
+                        out.stride(0), _p(addend), ldd, _p(bias), M, N, K, w.scales.data_ptr(), w.scales.stride(0))
+        check(load().dt_gemm_bf16_ws(ctypes.byref(p), io_type(out), _p(ws), ws.numel(), stream()), "dt_gemm_q8_0")
+        return out
     check(load().dt_gemm_q8_0(_p(a), a.stride(0), _p(w.codes), w.codes.stride(0), _p(w.scales),
                               w.scales.stride(0), _p(out), out.stride(0), M, N, K, _p(bias), _p(addend), ldd,
                               io_type(out), stream()), "dt_gemm_q8_0")
@@ -654,6 +676,12 @@ def gemm_f32(a, b, bias=None, addend=None, out=None):
     if out is None:
         out = torch.empty((M, N), dtype=torch.float32, device=a.device)
     ldd = addend.stride(0) if addend is not None else 0
+    ws = _gemm_ws(load().dt_gemm_f32_workspace_bytes, M, N, K, a)
+    if ws is not None:
+        p = GemmProblem(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), out.data_ptr(), out.stride(0),
+                        _p(addend), ldd, _p(bias), M, N, K, None, 0)
+        check(load().dt_gemm_f32_ws(ctypes.byref(p), _p(ws), ws.numel(), stream()), "dt_gemm_f32")
+        return out
     check(load().dt_gemm_f32(_p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0), M, N, K, _p(bias),
                              _p(addend), ldd, stream()), "dt_gemm_f32")
     return out

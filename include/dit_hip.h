@@ -433,6 +433,18 @@ int dt_flash_attn_qk_bf16(const void *q0, const int64_t *q0_strides, const float
 int dt_gemm_f32(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int64_t M,
                 int64_t N, int64_t K, const float *bias, const float *addend, int64_t ldd, dt_stream_t stream);
 int dt_gemm_f32_grouped(const dt_gemm_problem *problems, int32_t count, dt_stream_t stream);
+
+/* One product (bf16 or Q8_0 weights; fp32) that may be taken over several
+ * ranges of K at once, with their fp32 partial sums in `workspace` and added in
+ * range order by a second launch: for products with too few tiles to fill the
+ * GPU.  *_workspace_bytes: the bytes it then needs (16-byte aligned), 0 for a
+ * product that is not split; with less, or none, the call is dt_gemm_bf16's /
+ * dt_gemm_q8_0's / dt_gemm_f32's. */
+size_t dt_gemm_bf16_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int dt_gemm_bf16_ws(const dt_gemm_problem *problem, int32_t c_type, void *workspace, size_t workspace_bytes,
+                    dt_stream_t stream);
+size_t dt_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int dt_gemm_f32_ws(const dt_gemm_problem *problem, void *workspace, size_t workspace_bytes, dt_stream_t stream);
 size_t dt_flash_attn_f32_workspace_bytes(int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_kv,
                                          int64_t head_dim);
 int dt_flash_attn_f32(const float *q, const float *k, const float *v, float *o, int64_t batch, int64_t heads,

@@ -282,6 +282,38 @@ def test_gemm_q8_0_rejects(orc, dev):
                                  config=config)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("weights", ["bf16", "q8_0"])
+@pytest.mark.parametrize("M,N,K", [(1, 257, 4160), (16, 4100, 320), (7, 16400, 64),         # few rows, four or eight waves
+                                   (17, 5200, 256), (250, 3204, 448), (513, 4100, 320),     # two k-groups, odd k-tiles
+                                   (17, 516, 2112), (300, 253, 4160), (130, 2050, 576)])    # K ranges, ragged
+def test_gemm_few_tiles(orc, dev, M, N, K, weights, out_dtype):
+    """Products of few rows or few tiles, through gemm / gemm_q8_0 (K ranges with
+    a workspace) and the grouped call (none), with bias, addend and strides."""
+    print(f"few tiles {weights} {M}x{N}x{K} {out_dtype}", flush=True)
+    a, b = orc.randn(SEED + 270, (M, K + 8)), orc.randn(SEED + 271, (N, K), std=0.02)
+    bias, add = orc.randn(SEED + 272, (N,), std=0.1), orc.randn(SEED + 273, (M, N))
+    x = dev_tensor(a, torch.bfloat16)[:, :K]
+    if weights == "q8_0":
+        blocks = dit_hip.quantize_q8_0(dev_tensor(b, torch.float32))
+        w = dit_hip.q8_0_split(blocks.view(-1), N, K)
+        bw = host(dit_hip.dequant(blocks.view(-1), dit_hip.Q8_0, N, K, torch.bfloat16))
+        fn = dit_hip.gemm_q8_0
+    else:
+        w, bw, fn = dev_tensor(b, torch.bfloat16), orc.round_bf16(b), dit_hip.gemm
+    ld = (N + 3) // 4 * 4 + 4
+    out = torch.zeros((M, ld), dtype=out_dtype, device="cuda")
+    fn(x, w, bias=dev_tensor(bias, torch.float32), addend=dev_tensor(add, out_dtype), out=out[:, :N])
+    out2 = torch.empty((M, N), dtype=out_dtype, device="cuda")
+    dit_hip.gemm_grouped([(x, w, out2)])
+    torch.cuda.synchronize()
+    lin = orc.linear(orc.round_bf16(a[:, :K]), bw)
+    got = host(out)
+    check(got[:, :N], lin + bias + as_input(add, out_dtype), out_dtype, f"few tiles {M}x{N}x{K}")
+    assert not got[:, N:].any(), "wrote past N"
+    check(host(out2), lin, out_dtype, f"few tiles grouped {M}x{N}x{K}")
+
+
 # ---------------------------------------------------------------- attention --
 def _attn_ref(orc, q, k, v, scale=None):
     """q [B, Sq, H, D] -> oracle attention per batch on the bf16-rounded values."""
@@ -294,7 +326,7 @@ ATTN_SHAPES = [(1, 300, 300, 3), (2, 128, 64, 2), (1, 77, 500, 1), (1, 64, 1, 2)
 
 # ------------------------------------------------------------- fp32 path --
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (130, 200, 320), (256, 256, 3072), (77, 33, 40), (300, 136, 3),
-                                   (129, 260, 12288)])
+                                   (129, 260, 12288), (3, 16400, 128), (16, 100, 3072), (32, 68, 176), (17, 130, 2112)])
 def test_gemm_f32(orc, dev, M, N, K):
     """F32 weights with F32 activations (the reference's own Linear precision)
     in exact bf16 parts, against the oracle's linear at the fp32 bar
