@@ -423,12 +423,16 @@ __global__ __launch_bounds__(256) void conv2d_kernel(const ConvArgs a) {
 // multiple of 16 (to_nhwc16_kernel, one bandwidth-bound pass, which can also
 // apply a GroupNorm + SiLU), so a 16-channel slice of one pixel is a
 // contiguous 32-byte record and both operands stream into LDS by
-// global_load_lds with no per-element work: the input patch of a 256- or
+// global_load_lds with no per-element work: the input patch of a 128-, 256- or
 // 512-pixel tile (every lane computes its own source pixel, which also
 // applies the nearest 2x upscale and sends out-of-image taps to a zeroed
 // 256-byte tail of the workspace) and the [128 co][K*K] weight records.  Two
-// LDS stages of 16 channels, filled one chunk ahead; four waves of 64 co x
-// 32 FN px (2 x FN MFMA 32x32x16 per tap).  The DMA source swaps each
+// LDS stages of 16 channels, filled one chunk ahead; eight waves (two per SIMD: one's
+// MFMAs cover the other's LDS reads and waits) of 64 co x 32 FN px (2 x FN MFMA 32x32x16 per tap).
+// Four waves of twice the pixels, one per SIMD, took 160 us instead of 126 at
+// [1,128,512,512] -> 128, 178 instead of 162 at [1,512,160,160] -> 512 and, with the
+// residual epilogue on 256 pixels, 187 instead of 130 at [1,128,512,512]; the
+// statistics epilogue, which adds its waves' sums in pairs, keeps them.  The DMA source swaps each
 // 32-byte record's two 16-byte units by the rule below (kSwzBit), so
 // consecutive records read distinct banks.  The output leaves through LDS
 // (conv_store_lds).
@@ -440,16 +444,14 @@ constexpr int kCi2 = 16, kRec2 = 32;
 // on bit 2 repeated banks every 8 records: SQ_LDS_BANK_CONFLICT was half of
 // SQ_LDS_IDX_ACTIVE.)
 constexpr int kSwzBit = 3;
-// DMA lanes per X stage: 2 per record, up to the 10 x 34 records of an
-// 8 x 32 tile (the 16 x 16 tile needs 18 x 18).  Lanes past the patch read
-// the zero tail, so the count is kept to the largest patch.
-constexpr int kXLanesMax3 = 3 * 256;
-static_assert(2 * (8 + 2) * (32 + 2) <= kXLanesMax3 && 2 * (16 + 2) * (16 + 2) <= kXLanesMax3,
-              "X DMA lanes must cover the 3x3 patch of every tile shape conv_geometry2 picks");
-// The same for the 512-pixel tiles (16 x 32, or 32 x 16 on narrow images).
-constexpr int kXLanesMax3x2 = 5 * 256;
-static_assert(2 * (16 + 2) * (32 + 2) <= kXLanesMax3x2 && 2 * (32 + 2) * (16 + 2) <= kXLanesMax3x2,
-              "X DMA lanes must cover the 3x3 patch of every 512-pixel tile");
+// DMA lanes per X stage: 2 per record, up to the largest patch of the tile
+// shapes conv_geometry2 picks (8 x 32 or 16 x 16 pixels; 16 x 32 or 32 x 16), in
+// whole instructions of `threads` lanes.  Lanes past the patch read the zero tail.
+constexpr int conv_patch_lanes(int px, int K) {
+    const int wide = (px / 32 + K - 1) * (32 + K - 1), tall = (px / 16 + K - 1) * (16 + K - 1);
+    return 2 * (wide > tall ? wide : tall);
+}
+constexpr int conv_dma_count(int lanes, int threads) { return (lanes + threads - 1) / threads; }
 
 // GroupNorm applied by the channel-last copy: (mean, rstd) per (n, group),
 // the per-channel affine (or null), cg channels per group, the SiLU flag.
@@ -538,31 +540,31 @@ __device__ __forceinline__ void conv_wait_vm() {
     __builtin_amdgcn_s_waitcnt((N_OUT & 15) | ((N_OUT >> 4) << 14) | 0x0F70);
 }
 
-// The epilogue of the DMA kernel's 128-channel x 256-pixel tile, through
-// LDS, in two passes over the accumulator halves j (64 output channels
+// The epilogue of the DMA kernel's 128-channel x PX-pixel tile, through LDS,
+// in two passes over the accumulator halves j (64 output channels
 // each).  Each lane parks its conv + bias values, rounded to T as the graph
-// stores the conv node, in LDS as [64 channels][256 pixels]; the block then
+// stores the conv node, in LDS as [64 channels][PX pixels]; the block then
 // writes the pass in 16-byte pieces along the image rows (the lanes' own
 // values would be 2-byte stores).  RES adds the residual epilogue of
 // ResnetBlock2D's `(input + hidden) / output_scale_factor`: per piece the
 // residual (loaded before the LDS stage, so its latency overlaps it), the
 // ADD rounded to T, the SCALE (res_mode 2), one store.  A piece is read and
 // written by one thread only, so the output may sit on the residual.
-// The epilogue's LDS: 64 output-channel rows of the tile's 64 FN pixels,
+// The epilogue's LDS: 64 output-channel rows of the tile's PX pixels,
 // padded by 8 elements; the DMA kernel's shared array is at least this large.
-template <int FN>
-constexpr int epi_stride() { return 64 * FN + 8; }
-template <typename T, int FN>
-constexpr int epi_lds_bytes() { return 64 * epi_stride<FN>() * (int)sizeof(T); }
+constexpr int epi_stride(int px) { return px + 8; }
+template <typename T>
+constexpr int epi_lds_bytes(int px) { return 64 * epi_stride(px) * (int)sizeof(T); }
 
-template <typename T, bool RES, int FN>
+template <typename T, bool RES, int FN, int NWV>
 __device__ __forceinline__ void conv_store_lds(const ConvArgs& a, const f32x16_t (&acc)[2][FN], uint8_t* smem,
                                                int co0, int oh0, int ow0, int wco, int wpx, int lrow, int g, int lt,
                                                int n) {
     constexpr int E = Io<T>::EPV;             // elements per 16-byte piece
-    constexpr int S = epi_stride<FN>();       // LDS row stride in elements (bank-spread rows)
-    constexpr int RP = 64 * FN / E;           // pieces per pixel row
-    constexpr int PIECES = 64 * RP / 256;     // pieces per thread and pass
+    constexpr int PX = 16 * FN * NWV, NT = 64 * NWV;
+    constexpr int S = epi_stride(PX);         // LDS row stride in elements (bank-spread rows)
+    constexpr int RP = PX / E;                // pieces per pixel row
+    constexpr int PIECES = 64 * RP / NT;      // pieces per thread and pass
     T* lds = reinterpret_cast<T*>(smem);
     const int tid = threadIdx.x, tcm = (1 << lt) - 1;
     const int64_t plane = (int64_t)a.Hs * a.Ws;
@@ -575,7 +577,7 @@ __device__ __forceinline__ void conv_store_lds(const ConvArgs& a, const f32x16_t
         uint4 rv[PIECES];
 #pragma unroll
         for (int k = 0; k < PIECES && RES; ++k) {
-            const int c = tid + 256 * k, pr = c / RP, px = (c % RP) * E;
+            const int c = tid + NT * k, pr = c / RP, px = (c % RP) * E;
             const int co = co0 + (pr >> 5) * 64 + 32 * j + (pr & 31);
             const int oh = oh0 + (px >> lt), ow = ow0 + (px & tcm);
             rv[k] = make_uint4(0, 0, 0, 0);
@@ -625,7 +627,7 @@ __device__ __forceinline__ void conv_store_lds(const ConvArgs& a, const f32x16_t
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < PIECES; ++k) {
-            const int c = tid + 256 * k, pr = c / RP, px = (c % RP) * E;
+            const int c = tid + NT * k, pr = c / RP, px = (c % RP) * E;
             const int co = co0 + (pr >> 5) * 64 + 32 * j + (pr & 31);
             const int oh = oh0 + (px >> lt), ow = ow0 + (px & tcm);
             if (co >= a.Co || oh >= a.Hs || ow >= a.Ws) continue;
@@ -663,28 +665,28 @@ __device__ __forceinline__ void conv_store_lds(const ConvArgs& a, const f32x16_t
     }
 }
 
-// FN: 32-pixel MFMA columns per wave, 4 (a 256-pixel tile of 8 x 32) or 8
-// (512 pixels, 16 x 32, halving the weight DMA per output pixel, for convs
-// with enough tiles to fill the chip).
-template <typename T, int K, bool STATS, bool RES, int FN>
-__global__ __launch_bounds__(256) void conv2d_dma_kernel(const ConvArgs a, const Conv2Extra e) {
+// FN 32-pixel MFMA columns per wave, NWV waves (two of 64 channels by NWV / 2 along
+// the pixels): PX = 16 FN NWV pixels.
+template <typename T, int K, bool STATS, bool RES, int FN, int NWV>
+__global__ __launch_bounds__(64 * NWV) void conv2d_dma_kernel(const ConvArgs a, const Conv2Extra e) {
     static_assert(K == 3 || K == 1, "the DMA kernel takes 3x3 and 1x1 patches");
-    static_assert(FN == 4 || (FN == 8 && !STATS && !RES), "512-pixel tiles carry no statistics or residual epilogue");
+    static_assert(!STATS || NWV == 4, "the statistics epilogue pairs the waves of a 256-pixel tile");
     constexpr int KK = K * K, PAD = (K - 1) / 2;
-    constexpr int XL = FN == 4 ? kXLanesMax3 : kXLanesMax3x2;  // X DMA lanes per stage
-    constexpr int NX = XL / 256, NW = 2 * kTileCo * KK / 256;  // DMA instructions per wave per stage
-    constexpr int XB = XL * 16, WB = kTileCo * KK * kRec2, STAGE = XB + WB;
+    constexpr int PX = 16 * FN * NWV, NT = 64 * NWV;
+    // DMA instructions per wave per stage
+    constexpr int NX = conv_dma_count(conv_patch_lanes(PX, K), NT), NW = conv_dma_count(2 * kTileCo * KK, NT);
+    constexpr int XB = NX * NT * 16, WB = NW * NT * 16, STAGE = XB + WB;
     constexpr int QD = NX + NW;
     // the two DMA stages, then the epilogue's rows (larger for 1x1 patches)
-    constexpr int SMEM = 2 * STAGE > epi_lds_bytes<T, FN>() ? 2 * STAGE : epi_lds_bytes<T, FN>();
+    constexpr int SMEM = 2 * STAGE > epi_lds_bytes<T>(PX) ? 2 * STAGE : epi_lds_bytes<T>(PX);
     __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = blockIdx.z, co0 = blockIdx.y * kTileCo;
     const int th = blockIdx.x / a.tiles_w, tw = blockIdx.x - th * a.tiles_w;
     const int oh0 = th * a.TR, ow0 = tw * a.TC;
     const int PC = a.TC + K - 1, npatch = (a.TR + K - 1) * PC;
-    const int wco = (wave >> 1) * 64, wpx = (wave & 1) * 32 * FN;
+    const int wco = (wave / (NWV / 2)) * 64, wpx = (wave % (NWV / 2)) * 32 * FN;
     const int lrow = lane & 31, g = lane >> 5;
 
     // DMA sources, fixed for the whole K loop up to the channel offset.
@@ -692,7 +694,7 @@ __global__ __launch_bounds__(256) void conv2d_dma_kernel(const ConvArgs a, const
     int xstep[NX];  // 1 for an in-image record (advances with the channel chunk), 0 for the zero tail
 #pragma unroll
     for (int m = 0; m < NX; ++m) {
-        const int L = (m * 4 + wave) * 64 + lane, rec = L >> 1, u = L & 1;
+        const int L = (m * NWV + wave) * 64 + lane, rec = L >> 1, u = L & 1;
         const uint16_t* src = e.zero;
         xstep[m] = 0;
         if (rec < npatch) {
@@ -710,8 +712,9 @@ __global__ __launch_bounds__(256) void conv2d_dma_kernel(const ConvArgs a, const
     const uint16_t* wsrc[NW];
 #pragma unroll
     for (int m = 0; m < NW; ++m) {
-        const int L = (m * 4 + wave) * 64 + lane, rec = L >> 1, u = L & 1;
-        const int co = rec / KK, tap = rec - co * KK;
+        const int L = (m * NWV + wave) * 64 + lane, rec = L >> 1, u = L & 1;
+        // the last instruction's lanes past the tile's records load the last one again, past them
+        const int co = min(rec / KK, kTileCo - 1), tap = rec % KK;
         const int su = u ^ ((co >> kSwzBit) & 1);
         wsrc[m] = a.w + ((int64_t)(co0 + co) * KK + tap) * e.Cp32 + su * 8;
     }
@@ -719,9 +722,9 @@ __global__ __launch_bounds__(256) void conv2d_dma_kernel(const ConvArgs a, const
         uint8_t* st = smem + s * STAGE;
 #pragma unroll
         for (int m = 0; m < NX; ++m)  // out-of-image taps read the zero tail at every chunk
-            dma16(xsrc[m] + xstep[m] * c0, st + (m * 4 + wave) * 64 * 16);
+            dma16(xsrc[m] + xstep[m] * c0, st + (m * NWV + wave) * 64 * 16);
 #pragma unroll
-        for (int m = 0; m < NW; ++m) dma16(wsrc[m] + c0, st + XB + (m * 4 + wave) * 64 * 16);
+        for (int m = 0; m < NW; ++m) dma16(wsrc[m] + c0, st + XB + (m * NWV + wave) * 64 * 16);
     };
 
     f32x16_t acc[2][FN];
@@ -781,7 +784,7 @@ __global__ __launch_bounds__(256) void conv2d_dma_kernel(const ConvArgs a, const
 
     // The stores go through LDS (ending in a barrier, so the statistics
     // below may reuse it).
-    conv_store_lds<T, RES, FN>(a, acc, smem, co0, oh0, ow0, wco, wpx, lrow, g, e.lt, n);
+    conv_store_lds<T, RES, FN, NWV>(a, acc, smem, co0, oh0, ow0, wco, wpx, lrow, g, e.lt, n);
     if constexpr (STATS) {
         float* red = reinterpret_cast<float*>(smem);
         switch (a.cg) {
@@ -792,6 +795,109 @@ __global__ __launch_bounds__(256) void conv2d_dma_kernel(const ConvArgs a, const
             default: conv_group_stats_reg<T, 64, 4>(a, acc, red, co0, oh0, ow0, wco, wpx, lrow, g, wave); break;
         }
     }
+}
+
+// ---- 1x1 on bf16, straight from NCHW --------------------------------------------
+// A 1x1 conv is bound by reading x and writing y ([1, 256, 512, 512] -> 128: 201 MB,
+// 39 us at 5.1 TB/s); through the channel-last copy it read x, wrote and read the copy
+// and took 138 us.  Here the [32 channels][256 pixels] slices of x stream into LDS as
+// they lie, whole 512-byte rows, and the MFMA's pixel operand is read from them
+// transposed (ds_read_tr16_b64: lane i of a 16-lane group gets four channels of pixel
+// i), so x is read once per 128 output channels and nothing else is written.
+// Eight waves of 64 channels x 64 pixels; three stages of 24 KB, two in flight, and two
+// workgroups per CU.  The channels are summed in the same order as through the
+// copy (k-steps of 16, ascending): the same bits.
+// X stage: the 32-byte pair q of row r at q ^ (r & 3), so a transposed read's four rows
+// hit distinct banks.  W stage: 16-byte chunk c of row r (64 bytes) at c ^ ((r >> 1 ^ r >>
+// 2) & 3).
+typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) short4_t* lds_short4_p;
+constexpr int kPwPx = 256, kPwCi = 32 /* conv_is_direct's */, kPwX = kPwCi * kPwPx * 2, kPwW = kTileCo * kPwCi * 2;
+constexpr int kPwStage = kPwX + kPwW, kPwStages = 3;
+
+template <bool RES>
+__global__ __launch_bounds__(512, 4) void conv1x1_kernel(const ConvArgs a, int64_t HW) {
+    constexpr int FN = 2, NWV = 8;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kPwStages * kPwStage];
+    static_assert(epi_lds_bytes<bf16>(kPwPx) <= kPwStages * kPwStage, "the epilogue's rows");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = blockIdx.z, co0 = blockIdx.y * kTileCo;
+    const int64_t p0 = (int64_t)blockIdx.x * kPwPx;
+    const int wco = (wave >> 2) * 64, wpx = (wave & 3) * 64;
+    const int lrow = lane & 31, g = lane >> 5;
+
+    // DMA: X in two instructions a wave (2 rows each), W in one (16 rows).
+    // Pixels past the plane load its last 8 (never stored).
+    const uint16_t* xsrc[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const int r = (m * NWV + wave) * 2 + (lane >> 5), c = lane & 31;
+        const int64_t px = p0 + ((((c >> 1) ^ (r & 3)) << 1) + (c & 1)) * 8;
+        xsrc[m] = reinterpret_cast<const uint16_t*>(a.x) + ((int64_t)n * a.Ci + r) * HW + (px < HW ? px : HW - 8);
+    }
+    const int wr = wave * 16 + (lane >> 2);
+    const uint16_t* wsrc = a.w + (int64_t)(co0 + wr) * a.Ci_pad + (((lane & 3) ^ (((wr >> 1) ^ (wr >> 2)) & 3)) << 3);
+    auto issue = [&](int ch, int s) {
+        uint8_t* st = smem + s * kPwStage;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) dma16(xsrc[m] + (int64_t)ch * kPwCi * HW, st + (m * NWV + wave) * 1024);
+        dma16(wsrc + ch * kPwCi, st + kPwX + wave * 1024);
+    };
+
+    f32x16_t acc[2][FN];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[j][i][q] = 0.f;
+    // Transposed reads: lane s of 16-lane group gi addresses row 8 g + s / 4 (+ 4), pixels
+    // 32 i + 16 (gi & 1) + 4 (s % 4) of the wave's 64.
+    const int s16 = lane & 15, trow = 8 * g + (s16 >> 2);
+    int xofs[FN];
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+        const int pair = (wpx >> 4) + 2 * i + ((lane >> 4) & 1);
+        xofs[i] = trow * kPwPx * 2 + ((pair ^ (trow & 3)) << 5) + 8 * (s16 & 3);
+    }
+    const int wsw = ((lrow >> 1) ^ (lrow >> 2)) & 3;
+    auto tr = [](const uint8_t* p) {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_p)(p)));
+    };
+    const int nch = a.Ci / kPwCi;
+    issue(0, 0);
+    if (nch > 1) issue(1, 1);
+    int st = 0;
+    for (int ch = 0; ch < nch; ++ch) {
+        if (ch + 1 < nch) conv_wait_vm<3>();
+        else conv_wait_vm<0>();
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the stage refilled next
+        __builtin_amdgcn_s_barrier();
+        if (ch + 2 < nch) issue(ch + 2, st == 0 ? 2 : st - 1);
+        const uint8_t* X = smem + st * kPwStage;
+        const uint8_t* W = X + kPwX;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            bf16x8_t wf[2], xf[FN];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                wf[j] = *reinterpret_cast<const bf16x8_t*>(W + (wco + 32 * j + lrow) * 64 + (((2 * kk + g) ^ wsw) << 4));
+#pragma unroll
+            for (int i = 0; i < FN; ++i) {
+                const uint2 lo = tr(X + xofs[i] + 16 * kk * kPwPx * 2);
+                const uint2 hi = tr(X + xofs[i] + (16 * kk + 4) * kPwPx * 2);
+                xf[i] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < FN; ++i)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], xf[i], acc[j][i], 0, 0, 0);
+        }
+        st = st == kPwStages - 1 ? 0 : st + 1;
+    }
+    __syncthreads();  // the epilogue reuses the stages
+    conv_store_lds<bf16, RES, FN, NWV>(a, acc, smem, co0, 0, (int)p0, wco, wpx, lrow, g, __builtin_ctz(kPwPx), n);
 }
 
 // Repack [Co][Ci][K][K] (fp32 or bf16) to bf16 [Co_pad][K*K][Ci_pad], zeros
@@ -909,24 +1015,42 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
     DT_REQUIRE(!gn || (fold->gn_groups > 0 && Ci % fold->gn_groups == 0 && !stats),
                "%s: the GroupNorm fold needs groups dividing the input channels", what);
     // With a workspace 3x3 convs, and 1x1 convs on bf16, take the DMA path
-    // (gfx950, 1x1 [1, 256, 512, 512] -> 128: bf16 158 us against 217 us
-    // staged; fp32 163 us against 136 us, its channel-last copy reading
-    // twice the bytes).
+    // (gfx950, 1x1 [1, 256, 512, 512] -> 128: bf16 49 us direct and 105 us through
+    // the channel-last copy against 217 us staged; fp32 163 us through the copy, reading
+    // twice the bytes, against 136 us staged).
     const bool dma = conv_uses_dma(K, io_type) && ws && ws_bytes >= (size_t)(nhwc_elems(N, Ci, H, W) * 2 + 256) &&
                      aligned16(ws) && (!stats || (a.cg >= 4 && a.cg <= 64));
     int64_t tiles_w, tiles_h;
     DT_REQUIRE(!gn || dma, "%s: the GroupNorm fold needs a 3x3 conv with a workspace", what);
-    // 512-pixel tiles (half the weight DMA per output pixel) when they still
-    // give two workgroups per CU; statistics and the residual epilogue keep
-    // 256-pixel tiles (their registers would spill with 256 accumulators).
-    int fn = 4;
-    if (dma && !stats && !res_mode) {
-        int tr, tc;
-        int64_t tw, th;
-        conv_geometry2(Hs, Ws, 512, &tr, &tc, &tw, &th);
-        if (tw * th * ((Co + kTileCo - 1) / kTileCo) * N >= 512) fn = 8;
+    if (dma && !stats && conv_is_direct(K, io_type, upscale2, x, N, Ci, H * W, y, Co)) {
+        // One row of H W pixels (a 1x1 conv has no rows of its own).
+        a.TR = 1;
+        a.TC = kPwPx;
+        a.Hs = 1;
+        a.Ws = (int)(H * W);
+        const dim3 g1((unsigned)((H * W + kPwPx - 1) / kPwPx), (unsigned)((Co + kTileCo - 1) / kTileCo), (unsigned)N);
+        *n_tiles = g1.x;
+        if (res_mode) hipLaunchKernelGGL(conv1x1_kernel<true>, g1, dim3(512), 0, st, a, H * W);
+        else hipLaunchKernelGGL(conv1x1_kernel<false>, g1, dim3(512), 0, st, a, H * W);
+        return check_launch(what);
     }
-    if (dma) conv_geometry2(Hs, Ws, 64 * fn, &a.TR, &a.TC, &tiles_w, &tiles_h);
+    // The largest pixel tile that still gives every CU a workgroup (half the
+    // weight DMA per output pixel for each doubling), by tiles of the whole launch:
+    // 512 pixels from one per CU ([1,256,256,256] -> 256, 256 tiles: 95 us against 106
+    // at 256 pixels), 256 from more than one per two CUs, else 128
+    // ([1,512,64,64] -> 512, 64 tiles of 256: 55 us against 73; [1,512,32,32]: 51 and 68).
+    int px = 256;
+    if (dma && !stats) {
+        auto tiles = [&](int p) {
+            int tr, tc;
+            int64_t tw, th;
+            conv_geometry2(Hs, Ws, p, &tr, &tc, &tw, &th);
+            return tw * th * ((Co + kTileCo - 1) / kTileCo) * N;
+        };
+        const int cus = cu_count();
+        px = tiles(512) >= cus ? 512 : tiles(256) > cus / 2 ? 256 : 128;
+    }
+    if (dma) conv_geometry2(Hs, Ws, px, &a.TR, &a.TC, &tiles_w, &tiles_h);
     else conv_geometry(Hs, Ws, &a.TR, &a.TC, &tiles_w, &tiles_h);
     a.tiles_w = (int)tiles_w;
     DT_REQUIRE(tiles_h * tiles_w < (1ll << 31), "%s: too many tiles", what);
@@ -964,12 +1088,14 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
 #undef DT_NHWC
         int rc = check_launch(what);
         if (rc) return rc;
-#define DT_CONV2_LAUNCH(TT, KS, ST, RS)                                                                     \
-    do {                                                                                                    \
-        if (fn == 8)                                                                                        \
-            hipLaunchKernelGGL((conv2d_dma_kernel<TT, KS, ST, RS, ((ST || RS) ? 4 : 8)>), grid, dim3(256), 0, st, a, e); \
-        else                                                                                                \
-            hipLaunchKernelGGL((conv2d_dma_kernel<TT, KS, ST, RS, 4>), grid, dim3(256), 0, st, a, e);       \
+#define DT_CONV2_ONE(TT, KS, ST, RS, FN, NWV) \
+    hipLaunchKernelGGL((conv2d_dma_kernel<TT, KS, ST, RS, FN, NWV>), grid, dim3(64 * NWV), 0, st, a, e)
+#define DT_CONV2_LAUNCH(TT, KS, ST, RS)                          \
+    do {                                                         \
+        if (ST) DT_CONV2_ONE(TT, KS, ST, RS, 4, 4);              \
+        else if (px == 512) DT_CONV2_ONE(TT, KS, false, RS, 4, 8); \
+        else if (px == 256) DT_CONV2_ONE(TT, KS, false, RS, 2, 8); \
+        else DT_CONV2_ONE(TT, KS, false, RS, 1, 8);              \
     } while (0)
         if (io_type == DT_TYPE_F32) {
             if (K == 1) {
@@ -993,6 +1119,7 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
             }
         }
 #undef DT_CONV2_LAUNCH
+#undef DT_CONV2_ONE
         return check_launch(what);
     }
 #define DT_CONV_LAUNCH(TT, KS)                                                                         \

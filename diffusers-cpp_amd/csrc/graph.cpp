@@ -1155,7 +1155,10 @@ int run_conv(dt_backend* be, const dt_tensor* root, const dt_tensor* x, const dt
         const int rc = dt_conv2d_pack_weights(data_of(w), w->type, Co, Ci, K, scratch, st);
         if (rc) return rc;
     }
-    g_kernels += (prepacked ? 0 : 1) + (conv_uses_dma(K, root->type) ? 1 : 0) + 1;  // pack, channel-last copy, conv
+    // pack, channel-last copy, conv
+    const bool copies = conv_uses_dma(K, root->type) &&
+                        !conv_is_direct(K, root->type, up2, data_of(x), N, Ci, H * W, root->data, Co);
+    g_kernels += (prepacked ? 0 : 1) + (copies ? 1 : 0) + 1;
     const float* b = bias ? (const float*)data_of(bias) : nullptr;
     void* wsp = ws ? (char*)scratch + packed : nullptr;
     if (!res && !G) return dt_conv2d(data_of(x), N, Ci, H, W, wp, Co, K, up2, b, root->data, wsp, ws, root->type, st);

@@ -103,6 +103,18 @@ int backend_rope_table(dt_backend* be, int axis_dim, float freq_base, const floa
 // the channel-last copy and the DMA kernel (else the register-staged kernel).
 inline bool conv_uses_dma(int64_t K, int32_t io_type) { return K == 3 || (K == 1 && io_type == DT_TYPE_BF16); }
 
+// Whether such a conv, without statistics, is a 1x1 on bf16 read straight from
+// NCHW (conv1x1_kernel: whole 32-channel slices of 16-byte pixel groups), without
+// a channel-last copy.  A y that overlaps x keeps the copy, and so do planes under
+// 1024 pixels, where its launch is all there is to win ([1, 256, 16, 20] -> 128 18.7 us
+// against 16.0) and the launches a block reports stay as they were.
+inline bool conv_is_direct(int64_t K, int32_t io_type, int32_t upscale2, const void* x, int64_t N, int64_t Ci,
+                           int64_t HW, const void* y, int64_t Co) {
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+    return K == 1 && io_type == DT_TYPE_BF16 && !upscale2 && HW >= 1024 && Ci % 32 == 0 && HW % 8 == 0 && xa % 16 == 0 &&
+           (ya + (uintptr_t)(N * Co * HW) * 2 <= xa || xa + (uintptr_t)(N * Ci * HW) * 2 <= ya);
+}
+
 // Work the graph executor folds into a dt_conv2d (+ bias) launch
 // (conv2d.hip: conv2d_fold).
 struct ConvFold {

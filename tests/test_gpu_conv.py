@@ -354,8 +354,8 @@ def test_groupnorm_folded_into_conv_equals_the_nodes(orc, dev, io, shape, G, co,
     check(host(fused_out), want, io, "GroupNorm + conv", one_rounding=False)
 
 
-# 512-pixel tiles (16 x 32) are taken when they still give two workgroups
-# per CU (N x tiles x output-channel tiles >= 512); these shapes reach them,
+# 512-pixel tiles (16 x 32) are taken when they still give every CU a workgroup
+# (N x tiles x output-channel tiles >= 256); these shapes reach them,
 # with a batch, a partial output-channel tile, a partial column tile and the
 # 2x upscale.
 @pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
@@ -371,3 +371,42 @@ def test_conv2d_512_pixel_tiles(orc, dev, shape, co, up2, io):
     torch.cuda.synchronize()
     ref = orc.conv2d(orc.round_bf16(as_input(x, io)), orc.round_bf16(w), b, up2=up2)
     check(host(y), ref, io, f"conv2d 512px {shape} -> {co}")
+
+
+# The pixel tiles of the launch rule and the direct 1x1, at ragged edges, plain
+# and with the residual epilogue: the values a 256-CU card picks 512, 256 and
+# 128 pixels at, and 1x1 planes that end inside a 256-pixel tile.
+@pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape,co,k", [((1, 32, 270, 266), 200, 3), ((1, 32, 150, 133), 130, 3),
+                                        ((1, 48, 37, 30), 140, 3), ((2, 32, 36, 30), 130, 1), ((1, 96, 29, 40), 128, 1),
+                                        ((1, 32, 1, 1032), 4, 1)])
+def test_conv2d_tiles_and_residual(orc, dev, shape, co, k, io):
+    from graphkit import Backend
+    print(f"conv2d tiles x={shape} co={co} k={k} {io}", flush=True)
+    x = orc.randn(SEED + 93, shape)
+    w = orc.randn(SEED + 94, (co, shape[1], k, k), std=0.1)
+    b = orc.randn(SEED + 95, (co,), std=0.1)
+    res = orc.randn(SEED + 96, (shape[0], co, shape[2], shape[3]))
+    wp = dit_hip.conv2d_pack(dev_tensor(w, torch.float32))
+    y = dit_hip.conv2d(dev_tensor(x, io), wp, bias=dev_tensor(b, torch.float32), workspace=True)
+    staged = dit_hip.conv2d(dev_tensor(x, io), wp, bias=dev_tensor(b, torch.float32), workspace=None)
+    be = Backend()
+    try:
+        g, _, yn, out = _residual_graph(x, w, b, res, 0.5, io, True)
+        g.compute(be.h, outputs=[yn])
+        torch.cuda.synchronize()
+    finally:
+        be.close()
+    ref = orc.conv2d(orc.round_bf16(as_input(x, io)), orc.round_bf16(w), b)
+    check(host(y), ref, io, f"conv2d {shape} -> {co}")
+    check(host(staged), ref, io, f"conv2d staged {shape} -> {co}")
+    check(host(out), (as_input(res, io) + ref) * np.float32(0.5), io, "conv + residual", one_rounding=False)
+
+
+def test_conv2d_1x1_in_place(orc, dev):
+    """y over x: the 1x1 keeps its channel-last copy."""
+    x, w = orc.randn(SEED + 97, (1, 160, 32, 40)), orc.randn(SEED + 98, (160, 160, 1, 1), std=0.1)
+    xd = dev_tensor(x, torch.bfloat16)
+    dit_hip.conv2d(xd, dit_hip.conv2d_pack(dev_tensor(w, torch.float32)), out=xd)
+    torch.cuda.synchronize()
+    check(host(xd), orc.conv2d(orc.round_bf16(x), orc.round_bf16(w), None), torch.bfloat16, "1x1 in place")
