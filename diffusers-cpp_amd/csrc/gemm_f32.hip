@@ -41,7 +41,8 @@
 // a part of them falls below bf16's range and it would show) send their tile
 // through the fp32 matrix cores instead (f32_tile_native).
 //
-// Attention (no mask, head_dim 128): per (batch, head), S = Q K^T by the
+// Attention (no mask) for head dims other than 128 or rows that are not 16-byte aligned
+// (the others run attention_f32.hip's fused kernel): per (batch, head), S = Q K^T by the
 // GEMM, P = softmax(scale S) row by row in fp32 (max, then expf(scale s - max),
 // then the sum), O = P V by the GEMM against V^T (a transposed copy), heads
 // taken eight at a time through a workspace -- the fp32 arithmetic of ggml's
@@ -701,7 +702,8 @@ extern "C" int dt_gemm_f32_ws(const dt_gemm_problem* problem, void* workspace, s
 }
 
 // Workspace of dt_flash_attn_f32: per head of a group of up to 8, the
-// scores [seq_q][seq_kv] and V^T [head_dim][seq_kv], fp32.
+// scores [seq_q][seq_kv] and V^T [head_dim][seq_kv], fp32; or what the fused kernel
+// needs, if that is more.
 static int64_t attn_f32_group(int64_t batch, int64_t heads) {
     const int64_t bh = batch * heads;
     return bh < dit::kF32MaxGroup ? bh : dit::kF32MaxGroup;
@@ -711,7 +713,9 @@ extern "C" size_t dt_flash_attn_f32_workspace_bytes(int64_t batch, int64_t heads
                                                      int64_t head_dim) {
     if (batch <= 0 || heads <= 0 || seq_q <= 0 || seq_kv <= 0 || head_dim <= 0) return 0;
     const int64_t per = (seq_q * seq_kv + head_dim * seq_kv + 3) / 4 * 4;  // 16-byte aligned per head
-    return (size_t)(attn_f32_group(batch, heads) * per) * sizeof(float);
+    const size_t gemms = (size_t)(attn_f32_group(batch, heads) * per) * sizeof(float);
+    const size_t fused = head_dim == 128 ? dit::attn_f32_fused_bytes(batch, heads, seq_q, seq_kv) : 0;
+    return gemms > fused ? gemms : fused;
 }
 
 extern "C" int dt_flash_attn_f32(const float* q, const float* k, const float* v, float* o, int64_t batch,
@@ -731,6 +735,10 @@ extern "C" int dt_flash_attn_f32(const float* q, const float* k, const float* v,
     DT_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
                "dt_flash_attn_f32: workspace of %zu bytes (16-byte aligned) needed", need);
     hipStream_t st = (hipStream_t)stream;
+    if (attn_f32_fused_takes(q, k, v, o, batch, heads, seq_q, seq_kv, head_dim, q_strides, k_strides, v_strides, o_strides,
+                             scale))
+        return attn_f32_fused(q, k, v, o, batch, heads, seq_q, seq_kv, q_strides, k_strides, v_strides, o_strides, scale,
+                              workspace, st);
     const int64_t per = (seq_q * seq_kv + head_dim * seq_kv + 3) / 4 * 4;
     const int64_t bh = batch * heads, gsz = attn_f32_group(batch, heads);
     float* ws = (float*)workspace;

@@ -423,6 +423,52 @@ def test_flash_attn_f32(orc, dev, B, Sq, Skv, H):
     assert_fp32(host(o), ref, what=f"attn_f32 {B}x{Sq}x{Skv}x{H}")
 
 
+@pytest.mark.parametrize("case", ["strided", "scale0", "peaked", "inf_q", "nan_k", "inf_v", "huge_v", "tiny_v", "zero_v"])
+@pytest.mark.parametrize("B,Sq,Skv,H", [(1, 130, 33, 2), (2, 40, 260, 1), (1, 33, 31, 2)])
+def test_flash_attn_f32_ranges(dev, B, Sq, Skv, H, case):
+    """Ragged tiles, one or more key ranges, strided rows, and operands outside
+    the range the fused kernel splits (their heads run in plain fp32): against 64
+    bits within 1e-5 of the largest |v| a row can meet, NaN rows the same."""
+    print(f"attn_f32 {case} B={B} Sq={Sq} Skv={Skv} H={H}", flush=True)
+    g = torch.Generator().manual_seed(SEED + Skv)
+    q, k, v = (torch.randn((B, S, H, 128), generator=g) for S in (Sq, Skv, Skv))
+    scale = {"scale0": 0.0, "peaked": 3.0}.get(case, 128 ** -0.5)
+    if case == "peaked":
+        k *= 30.0  # scores of thousands: one key's weight is 1, the reference moves
+    elif case == "inf_q":
+        q[0, 3, 0, 5] = float("inf")
+    elif case == "nan_k":
+        k[0, 7, H - 1, 0] = float("nan")
+    elif case == "inf_v":
+        v[0, 2, 0, 9] = float("-inf")
+    elif case == "huge_v":
+        v[:, :, 0] *= 2.0 ** 100
+    elif case == "tiny_v":
+        v[:, :, H - 1] *= 2.0 ** -110
+    elif case == "zero_v":
+        v.zero_()
+    big = torch.zeros((B, Sq, H, 132), device="cuda")
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    if case == "strided":
+        big[..., :128] = qd
+        qd = big[..., :128]
+    o = dit_hip.flash_attn_f32(qd, kd, vd, scale=scale)
+    torch.cuda.synchronize()
+    q, k, v = (t.double().permute(0, 2, 1, 3).contiguous() for t in (q, k, v))
+    s = (q @ k.transpose(-1, -2).contiguous()) * scale
+    ref = (torch.softmax(s, -1) @ v).permute(0, 2, 1, 3)
+    got = o.cpu().double()
+    nan = torch.isnan(ref)
+    assert torch.equal(torch.isnan(got), nan)
+    inf = torch.isinf(ref)
+    assert torch.equal(got[inf], ref[inf])
+    vmax = torch.where(torch.isfinite(v), v.abs(), 0.0).amax((2, 3))[:, None, :, None].expand(ref.shape)
+    ok = ~nan & ~inf
+    # a score's fp32 rounding, 2^-24 of 128 products' magnitudes, moves a weight by as much
+    smax = (q.abs() @ k.abs().transpose(-1, -2).contiguous()).nan_to_num(0.0, 0.0).amax().item() * scale
+    assert ((got - ref).abs()[ok] <= max(1e-5, 2.0 ** -23 * smax) * vmax[ok]).all()
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,Sq,Skv,H", ATTN_SHAPES)
 def test_flash_attn(orc, dev, B, Sq, Skv, H, out_dtype):
