@@ -82,100 +82,6 @@ __device__ __forceinline__ int pro_position(const RopeAxisPos& pos, int axis, in
     return p[(int64_t)t * st];
 }
 
-// Query `qrow` of the wave with QK-RMSNorm + RoPE applied, written as bf16
-// to `row` (256 bytes of LDS): lane half g owns dims 16 c + 8 g + [0, 8) of
-// chunk c, as in the B operand it is read back into.  Every operation is
-// the QK kernel's (qk_rope.hip), in its order: per 8-dim chunk the sum of
-// squares, the 16 chunk sums added as its 16-lane DPP tree does (pairs,
-// quads, halves, whole), 1 / sqrt(ss / 128 + eps), (x * r) * w, the
-// rotation, one bf16 rounding -- so the q used here is bit-identical to the
-// stored output of dt_qk_rmsnorm_rope.  The chunk loop writes LDS rather than
-// registers, so it need not unroll and adds nothing to the main loop's
-// register budget; the second pass re-reads the chunks (cache hits).
-__device__ __forceinline__ void q_prologue(const AttnPro& pro, int b, int h, int qrow, int seq_q, int g,
-                                           uint8_t* row) {
-    const bool valid = qrow < seq_q;
-    const int seg = valid && qrow >= pro.split;
-    const int tok = seg ? qrow - pro.split : qrow;
-    const uint16_t* src = seg ? pro.q1 + b * pro.q1_bs + (int64_t)tok * pro.q1_ts + h * pro.q1_hs
-                              : pro.q0 + b * pro.q0_bs + (int64_t)tok * pro.q0_ts + h * pro.q0_hs;
-    // Every independent load first: the positions (their table rows are the
-    // one dependent load), the 8 chunks of q.
-    int p[8];
-    bool hit = valid && pro.table != nullptr;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const int d0 = 16 * c + 8 * g;
-        p[c] = valid ? pro_position(pro.pos, d0 / pro.axis_dim, qrow) : 0;
-    }
-    uint4 raw[8];
-    float part[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) raw[c] = valid ? ld16(src + 16 * c + 8 * g) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) hit = hit && p[c] >= 0 && p[c] < pro.n_pos;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        float v[8];
-        Io<bf16>::unpack(raw[c], v);
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-        part[c] = ss;
-    }
-    // Chunk 2 c + g is here, 2 c + (1 - g) in lane l ^ 32: their sum is the
-    // tree's first level whichever half holds which.
-    float s1[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) s1[c] = part[c] + __shfl_xor(part[c], 32);
-    const float ss = ((s1[0] + s1[1]) + (s1[2] + s1[3])) + ((s1[4] + s1[5]) + (s1[6] + s1[7]));
-    const float r = 1.0f / sqrtf(ss / (float)D + pro.eps);
-    const float* w = seg ? pro.w1 : pro.w0;
-    auto emit = [&](int c, const float* v, const float* cs) {
-        const int d0 = 16 * c + 8 * g;
-        float wv[8], o[8];
-        const float4 wa = *reinterpret_cast<const float4*>(w + d0);
-        const float4 wb = *reinterpret_cast<const float4*>(w + d0 + 4);
-        wv[0] = wa.x; wv[1] = wa.y; wv[2] = wa.z; wv[3] = wa.w;
-        wv[4] = wb.x; wv[5] = wb.y; wv[6] = wb.z; wv[7] = wb.w;
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-            const float x0 = mul_rn(mul_rn(v[2 * qd], r), wv[2 * qd]);
-            const float x1 = mul_rn(mul_rn(v[2 * qd + 1], r), wv[2 * qd + 1]);
-            const float cn = cs[2 * qd], sn = cs[2 * qd + 1];
-            o[2 * qd] = sub_rn(mul_rn(x0, cn), mul_rn(x1, sn));
-            o[2 * qd + 1] = add_rn(mul_rn(x0, sn), mul_rn(x1, cn));
-        }
-        *reinterpret_cast<uint4*>(row + 2 * d0) = Io<bf16>::pack(o);
-    };
-    if (hit) {  // every angle from the table: unrolled, its loads issued together
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const int d0 = 16 * c + 8 * g;
-            const int i0 = d0 - (d0 / pro.axis_dim) * pro.axis_dim;
-            const float* t = pro.table + (int64_t)p[c] * pro.axis_dim + i0;  // rope_angles' table branch
-            const float4 ca = *reinterpret_cast<const float4*>(t), cb = *reinterpret_cast<const float4*>(t + 4);
-            const float cs[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
-            float v[8];
-            Io<bf16>::unpack(raw[c], v);
-            emit(c, v, cs);
-        }
-    } else if (valid) {  // some angle off the table: the device recurrence
-        for (int c = 0; c < 8; ++c) {
-            const int d0 = 16 * c + 8 * g;
-            const int axis = d0 / pro.axis_dim, i0 = d0 - axis * pro.axis_dim;
-            float cs[8], v[8];
-            rope_angles<4>(pro_position(pro.pos, axis, qrow), i0, pro.table, pro.n_pos, pro.axis_dim,
-                           pro.theta_scale, cs);
-            Io<bf16>::unpack(ld16(src + d0), v);
-            emit(c, v, cs);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) *reinterpret_cast<uint4*>(row + 2 * (16 * c + 8 * g)) = make_uint4(0, 0, 0, 0);
-    }
-}
-
 // ---- K/V by direct DMA, two workgroups per CU ---------------------------------
 // K and V tiles move global -> LDS by direct DMA (global_load_lds_dwordx4)
 // into two 32 KB buffers, so no registers are spent on staging.  At most 256 registers per lane (two waves per SIMD):
@@ -206,6 +112,45 @@ typedef __attribute__((address_space(3))) short4_t* lds_short4_p;
 // ds_read_tr16_b64 of the 8 bytes at p (an LDS address).
 __device__ __forceinline__ uint2 read_tr16(const uint8_t* p) {
     return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_p)(p)));
+}
+
+// Chunk c (8 dims) of query q0 + row with QK-RMSNorm + RoPE applied, 16 lanes a
+// query, as bf16 into row `row` of `rows` in LDS (chunk c at c ^ (row & 15)).  Every
+// operation is the QK kernel's (qk_rope.hip), in its order: per 8-dim chunk the sum of
+// squares, the 16 chunk sums added by its 16-lane DPP tree, 1 / sqrt(ss / 128 +
+// eps), (x * r) * w, the rotation, one bf16 rounding -- so the q used here is
+// bit-identical to the stored output of dt_qk_rmsnorm_rope.  (A lane taking half of a
+// query's chunks, as its MFMA operand holds them, made 16-byte loads of 64 scattered
+// lines and a long unrolled body: about 5 us of the 16.5 a 320-token attention took.)
+__device__ __forceinline__ void q_prologue16(const AttnPro& pro, int b, int h, int q0, int row, int seq_q, int c,
+                                             uint8_t* rows) {
+    const int qrow = min(q0 + row, seq_q - 1);  // rows past the sequence are never stored
+    const int seg = qrow >= pro.split, tok = seg ? qrow - pro.split : qrow;
+    const uint16_t* src = seg ? pro.q1 + b * pro.q1_bs + (int64_t)tok * pro.q1_ts + h * pro.q1_hs
+                              : pro.q0 + b * pro.q0_bs + (int64_t)tok * pro.q0_ts + h * pro.q0_hs;
+    const int d0 = 8 * c, axis = d0 / pro.axis_dim;
+    const int p = pro_position(pro.pos, axis, qrow);
+    const uint4 raw = ld16(src + d0);
+    const float* w = (seg ? pro.w1 : pro.w0) + d0;
+    const float4 wa = *reinterpret_cast<const float4*>(w), wb = *reinterpret_cast<const float4*>(w + 4);
+    const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
+    float cs[8], v[8], o[8];
+    rope_angles<4>(p, d0 - axis * pro.axis_dim, pro.table, pro.n_pos, pro.axis_dim, pro.theta_scale, cs);
+    Io<bf16>::unpack(raw, v);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+    ss = row16_sum(ss);
+    const float rs = 1.0f / sqrtf(ss / (float)D + pro.eps);
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+        const float x0 = mul_rn(mul_rn(v[2 * qd], rs), wv[2 * qd]);
+        const float x1 = mul_rn(mul_rn(v[2 * qd + 1], rs), wv[2 * qd + 1]);
+        const float cn = cs[2 * qd], sn = cs[2 * qd + 1];
+        o[2 * qd] = sub_rn(mul_rn(x0, cn), mul_rn(x1, sn));
+        o[2 * qd + 1] = add_rn(mul_rn(x0, sn), mul_rn(x1, cn));
+    }
+    *reinterpret_cast<uint4*>(rows + row * DROW + ((c ^ (row & 15)) << 4)) = Io<bf16>::pack(o);
 }
 
 template <typename TO, bool PRO>
@@ -404,11 +349,14 @@ __global__ __launch_bounds__(256, 2) void flash_attn_dma_kernel(AttnArgs a, Attn
         // tile's DMA (above) is in flight: wave w's rows at [32 w, 32 w +
         // 32) x 256 B.  Every wave has read its rows back before the
         // barrier, and the buffer's first DMA comes after it.
-        uint8_t* row = smem + 2 * DTILE + (32 * wave + r) * DROW;
-        q_prologue(pro, b, h, q0 + r, a.seq_q, g, row);
+        uint8_t* rows = smem + 2 * DTILE + 32 * wave * DROW;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            q_prologue16(pro, b, h, q0, 4 * i + (lane >> 4), a.seq_q, lane & 15, rows);
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's rows are in LDS
 #pragma unroll
-        for (int c = 0; c < 8; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(row + 2 * (16 * c + 8 * g));
+        for (int c = 0; c < 8; ++c)
+            qf[c] = *reinterpret_cast<const bf16x8_t*>(rows + r * DROW + (((2 * c + g) ^ (r & 15)) << 4));
         __syncthreads();
     }
     int t = 0;
@@ -445,6 +393,248 @@ __global__ __launch_bounds__(256, 2) void flash_attn_dma_kernel(AttnArgs a, Attn
                         make_uint2(pack_bf16x2(v4[0], v4[1]), pack_bf16x2(v4[2], v4[3]));
                 }
             }
+    }
+}
+
+// ---- few query blocks: 32 queries per workgroup, keys over its waves -------------
+// With blocks of 128 queries a short sequence or few heads leave most CUs idle (24
+// heads of 320 tokens: 72 workgroups), and each then walks all keys by itself.  Here
+// a workgroup takes 32 queries and each of its four waves every fourth 32-key tile, from
+// K and V buffers of its own (8 KB each): a wave waits only for its own DMA and there
+// is no barrier until the four partial results meet in LDS.  K of the wave's next
+// tile loads from the end of its scores on, V from the end of P V on.  The
+// products, the softmax and its moving reference are flash_attn_dma_kernel's.
+// Kernel time (launches in one HIP graph), against blocks of 128: 24 heads of 320 16.1
+// -> 8.9 us, of 20 8.7 -> 6.0, 8 heads of 1000 28.8 -> 15.7, 2 of 2048 45 -> 23; past two
+// workgroups per CU K and V are read too often (24 heads of 700, 528 workgroups: 24.8
+// against 34.7, of 1000 31 against 43, with the older prologue's 4 us).  Eight waves a
+// workgroup were slower (13.5 -> 15.8 us at 24 heads of 320).
+constexpr int NW = 4, FQB = 32, FKB = 32, FTILE = FKB * DROW;  // waves; 8 KB
+
+// The wave's 32 keys x 128 d of V as the V^T operands of both 16-key steps: lo, hi of
+// block tt and step j at vf[j][tt].  The wait is in the block, so nothing reads
+// the registers early; the compiler's own wait before its transposed reads would also
+// drain the DMA in flight.
+__device__ __forceinline__ void read_v_tile(uint32_t lds, const int (&voff)[4], bf16x8_t (&vf)[2][4]) {
+    uint2 r[2][4][2];
+    uint32_t at[4];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) at[tt] = lds + (uint32_t)voff[tt];
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16\n\t"
+        "ds_read_b64_tr_b16 %1, %16 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %2, %17\n\t"
+        "ds_read_b64_tr_b16 %3, %17 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %4, %18\n\t"
+        "ds_read_b64_tr_b16 %5, %18 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %6, %19\n\t"
+        "ds_read_b64_tr_b16 %7, %19 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %8, %16 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %9, %16 offset:6144\n\t"
+        "ds_read_b64_tr_b16 %10, %17 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %11, %17 offset:6144\n\t"
+        "ds_read_b64_tr_b16 %12, %18 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %13, %18 offset:6144\n\t"
+        "ds_read_b64_tr_b16 %14, %19 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %15, %19 offset:6144\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0][0][0]), "=&v"(r[0][0][1]), "=&v"(r[0][1][0]), "=&v"(r[0][1][1]), "=&v"(r[0][2][0]),
+          "=&v"(r[0][2][1]), "=&v"(r[0][3][0]), "=&v"(r[0][3][1]), "=&v"(r[1][0][0]), "=&v"(r[1][0][1]),
+          "=&v"(r[1][1][0]), "=&v"(r[1][1][1]), "=&v"(r[1][2][0]), "=&v"(r[1][2][1]), "=&v"(r[1][3][0]),
+          "=&v"(r[1][3][1])
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
+        : "memory");
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+            vf[j][tt] = __builtin_bit_cast(bf16x8_t, make_uint4(r[j][tt][0].x, r[j][tt][0].y, r[j][tt][1].x, r[j][tt][1].y));
+}
+
+template <typename TO, bool PRO>
+__global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, AttnPro pro) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NW * 2 * FTILE];  // [wave][K | V]
+    __shared__ __attribute__((aligned(16))) uint8_t qrows[PRO ? FTILE : 16];
+    __shared__ float ml[2][NW][FQB];
+    uint32_t bid = blockIdx.x;
+    const uint32_t nb = gridDim.x;
+    if ((nb & 7u) == 0) bid = (bid & 7u) * (nb >> 3) + (bid >> 3);
+    const int blocks = (a.seq_q + FQB - 1) / FQB;
+    const int qblk = (int)(bid % (uint32_t)blocks), bh = (int)(bid / (uint32_t)blocks);
+    const int h = bh % a.heads, b = bh / a.heads;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, g = lane >> 5, q = qblk * FQB + r;
+    const uint16_t* Kp = a.k + b * a.ks[0] + h * a.ks[2];
+    const uint16_t* Vp = a.v + b * a.vs[0] + h * a.vs[2];
+    uint8_t* const Kt = smem + wave * 2 * FTILE;
+    uint8_t* const Vt = Kt + FTILE;
+
+    // DMA: eight instructions of 4 rows; rows past seq_kv load the last one.
+    const int drow = lane >> 4, dpos = lane & 15;
+    auto issue = [&](const uint16_t* src, int64_t ts, int t, uint8_t* buf, auto is_k) {
+        const int k0 = t * FKB;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int row = 4 * j + drow, sw = decltype(is_k)::value ? kswz(row) : vswz(row);
+            __builtin_amdgcn_global_load_lds(src + min(k0 + row, a.seq_kv - 1) * ts + (dpos ^ sw) * 8, buf + 4 * j * DROW,
+                                             16, 0, 0);
+        }
+    };
+    auto issue_k = [&](int t) { issue(Kp, a.ks[1], t, Kt, std::true_type{}); };
+    auto issue_v = [&](int t) { issue(Vp, a.vs[1], t, Vt, std::false_type{}); };
+
+    const int ntiles = (a.seq_kv + FKB - 1) / FKB;
+    if (wave < ntiles) issue_k(wave);
+    // Each wave prepares eight of the block's queries for all.
+    bf16x8_t qf[8];
+    if constexpr (PRO) {
+#pragma unroll
+        for (int i = 0; i < FQB / (4 * NW); ++i)
+            q_prologue16(pro, b, h, qblk * FQB, (FQB / NW) * wave + 4 * i + (lane >> 4), a.seq_q, lane & 15, qrows);
+        // Not __syncthreads: K's DMA stays in flight.
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's rows are in LDS
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            qf[c] = *reinterpret_cast<const bf16x8_t*>(qrows + r * DROW + (((2 * c + g) ^ (r & 15)) << 4));
+    } else {
+        const uint16_t* Qp = a.q + b * a.qs[0] + h * a.qs[2];
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            qf[c] = __builtin_bit_cast(bf16x8_t, q < a.seq_q ? ld16(Qp + (int64_t)q * a.qs[1] + 16 * c + 8 * g)
+                                                             : make_uint4(0, 0, 0, 0));
+    }
+    if (wave < ntiles) issue_v(wave);
+
+    int koff[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) koff[c] = r * DROW + (((2 * c + g) ^ (r & 15)) << 4);
+    const int s16 = lane & 15, gi = lane >> 4, tg = gi >> 1, dsub = gi & 1;
+    const int trow = s16 >> 2, tcol = 16 * dsub + 4 * (s16 & 3);
+    int voff[4];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+        voff[tt] = (4 * tg + trow) * DROW + ((4 * (tt ^ trow) + (tcol >> 3)) << 4) + 8 * ((tcol >> 2) & 1);
+    const uint32_t vlds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)Vt;
+
+    f32x16_t o[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    const float sc = a.scale_log2;
+    for (int t = wave; t < ntiles; t += NW) {
+        attn_wait_vm<8>();  // K (V's eight are younger)
+        f32x16_t s[2];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[0][e] = s[1][e] = 0.f;
+        __builtin_amdgcn_sched_barrier(0);  // no LDS read before the wait
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(Kt + koff[c]);
+            s[c & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s[c & 1], 0, 0, 0);
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): K read, its buffer is free
+        __builtin_amdgcn_sched_barrier(0);
+        const bool more = t + NW < ntiles;
+        if (more) issue_k(t + NW);
+        // Element i is key 32 t + 8 (i / 4) + 4 g + i % 4.
+        const int left = a.seq_kv - t * FKB;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[0][i] += s[1][i];
+            if (8 * (i >> 2) + 4 * g + (i & 3) < left) mx = fmaxf(mx, s[0][i]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_cand = fmaxf(m_run, mx * sc);
+        const bool move = m_cand > m_run + 8.0f;
+        if (__builtin_amdgcn_ballot_w64(move)) {
+            const float m_new = move ? m_cand : m_run;
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            l_run *= alpha;
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[tt][e] *= alpha;
+            m_run = m_new;
+        }
+        float psum = 0.f;
+        bf16x8_t pf[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t pk[4];
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                float p2[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int i = 8 * j + e + u;
+                    float arg = __builtin_fmaf(s[0][i], sc, -m_run);
+                    if (8 * (i >> 2) + 4 * g + (i & 3) >= left) arg = -INFINITY;
+                    p2[u] = __builtin_amdgcn_exp2f(arg);
+                    psum += p2[u];
+                }
+                pk[e / 2] = pack_bf16x2(p2[0], p2[1]);
+            }
+            pf[j] = __builtin_bit_cast(bf16x8_t, make_uint4(pk[0], pk[1], pk[2], pk[3]));
+        }
+        l_run += psum;
+        if (more) attn_wait_vm<8>();  // V (K's next eight are younger)
+        else attn_wait_vm<0>();
+        bf16x8_t vf[2][4];
+        read_v_tile(vlds, voff, vf);
+        if (more) issue_v(t + NW);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt)
+                o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[j][tt], pf[j], o[tt], 0, 0, 0);
+    }
+
+    // The waves' results share the largest reference: O = sum w_i O_i / sum w_i l_i.
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    if (g == 0) {
+        ml[0][wave][r] = m_run;
+        ml[1][wave][r] = l_tot;
+    }
+    __syncthreads();
+    float m = ml[0][0][r];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m = fmaxf(m, ml[0][w][r]);
+    const float mine = __builtin_amdgcn_exp2f(m_run - m);
+    float* part = reinterpret_cast<float*>(smem);  // [wave][128 d][32 q]
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            part[wave * D * FQB + (32 * tt + 8 * (e >> 2) + 4 * g + (e & 3)) * FQB + r] = o[tt][e] * mine;
+    __syncthreads();
+    const int qq = qblk * FQB + r, d0 = (tid >> 5) * (64 / NW);
+    float l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) l += __builtin_amdgcn_exp2f(ml[0][w][r] - m) * ml[1][w][r];
+    const float inv = 1.0f / l;
+    if (qq < a.seq_q) {
+        TO* op = reinterpret_cast<TO*>(a.o) + b * a.os[0] + (int64_t)qq * a.os[1] + h * a.os[2];
+#pragma unroll
+        for (int d = d0; d < d0 + 64 / NW; d += 4) {
+            float v4[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = 0.f;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) v += part[w * D * FQB + (d + e) * FQB + r];
+                v4[e] = v * inv;
+            }
+            if constexpr (sizeof(TO) == 4)
+                *reinterpret_cast<float4*>(reinterpret_cast<float*>(op) + d) = make_float4(v4[0], v4[1], v4[2], v4[3]);
+            else
+                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(op) + d) =
+                    make_uint2(pack_bf16x2(v4[0], v4[1]), pack_bf16x2(v4[2], v4[3]));
+        }
     }
 }
 
@@ -496,8 +686,18 @@ int attn_prepare(const void* q, const void* k, const void* v, void* o, int64_t b
 
 template <bool PRO>
 int attn_launch(const AttnArgs& a, const AttnPro& pro, int32_t o_type, hipStream_t st, const char* who) {
-    const unsigned nblocks = (unsigned)((int64_t)a.q_blocks * a.heads * a.batch);
+    const int64_t blocks = (int64_t)a.q_blocks * a.heads * a.batch;
+    const unsigned nblocks = (unsigned)blocks;
     if (nblocks == 0) return DT_OK;
+    // Blocks of 32 queries while two per CU hold them all (see the kernel).
+    const int64_t few = (int64_t)((a.seq_q + FQB - 1) / FQB) * a.heads * a.batch;
+    if (few <= 2 * cu_count()) {
+        const dim3 grid((unsigned)few);
+        const bool f32 = o_type == DT_TYPE_F32;
+        if (f32) hipLaunchKernelGGL((flash_attn_few_kernel<float, PRO>), grid, dim3(64 * NW), 0, st, a, pro);
+        else hipLaunchKernelGGL((flash_attn_few_kernel<uint16_t, PRO>), grid, dim3(64 * NW), 0, st, a, pro);
+        return check_launch(who);
+    }
     if (o_type == DT_TYPE_F32)
         hipLaunchKernelGGL((flash_attn_dma_kernel<float, PRO>), dim3(nblocks), dim3(256), 0, st, a, pro);
     else

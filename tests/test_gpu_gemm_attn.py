@@ -593,6 +593,22 @@ def test_flash_attn_qk_prologue_bit_exact(orc, dev, B, n_txt, n_img, Skv, H, n_p
         assert_bf16(host(got)[0], ref, "attn+qk vs oracle")
 
 
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Sq,Skv,H", [(128, 97, 128), (129, 97, 128), (200, 64, 100), (1, 33, 2), (32, 128, 3),
+                                      (65, 161, 5)])
+def test_flash_attn_block_sizes(orc, dev, Sq, Skv, H, out_dtype):
+    """Both query block sizes (32 while 512 blocks hold the call on a 256-CU
+    card, 128 beyond) at the ends of their tiles, q as given and before its
+    QK-RMSNorm + RoPE (bit for bit the two-kernel path)."""
+    print(f"attn blocks Sq={Sq} Skv={Skv} H={H} {out_dtype}", flush=True)
+    n_txt = Sq // 3
+    test_flash_attn_qk_prologue_bit_exact(orc, dev, 1, n_txt, Sq - n_txt, Skv, H, 40, out_dtype)
+    q, k, v = (orc.randn(SEED + 249 + i, (1, S, H, 128)) for i, S in enumerate((Sq, Skv, Skv)))
+    o = dit_hip.flash_attn(*(dev_tensor(t, torch.bfloat16) for t in (q, k, v)), out_dtype=out_dtype)
+    torch.cuda.synchronize()
+    assert_bf16(host(o), _attn_ref(orc, q, k, v), "attention")
+
+
 def test_flash_attn_qk_prologue_flux2_shape(orc, dev):
     """A single-stream block's attention at 1024^2: q [4608, 24, 128] taken
     from the fused projection before its norm, 512 txt + 64x64 img positions,
