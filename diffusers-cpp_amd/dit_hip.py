@@ -10,6 +10,7 @@ ggml-ordered `dt_tensor` descriptor (ne[0] = last PyTorch dim).
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import POINTER, c_char_p, c_float, c_int32, c_int64, c_size_t, c_uint32, c_uint64, c_void_p
 
@@ -192,6 +193,7 @@ class _Recorder:
     def __init__(self, lib):
         self._lib = lib
         self.calls = []
+        self.keep = []  # scratch tensors the recorded calls point into
 
     def __getattr__(self, name):
         fn = getattr(self._lib, name)
@@ -224,12 +226,12 @@ def prepare(wrapper, *args, **kwargs):
     calls = rec.calls
     if len(calls) == 1:
         fn, conv = calls[0]
-        import functools
-        return result, functools.partial(fn, *conv)
-
-    def launch():
-        for fn, conv in calls:
-            fn(*conv)
+        launch = functools.partial(fn, *conv)
+    else:
+        def launch():
+            for fn, conv in calls:
+                fn(*conv)
+    launch.keep = rec.keep
     return result, launch
 
 
@@ -243,22 +245,41 @@ def check(rc: int, what: str = ""):
 # torch helpers
 # --------------------------------------------------------------------------
 
+# A small call's cost is this marshalling (17 us around a 9 us attention
+# kernel), so it is kept to lookups: torch and its dtype codes once, the raw
+# handle of the current stream, and stride triples (read only by the library).
+_TORCH = None
+_IO_TYPES = {}
+
+
 def _torch():
-    import torch
-    return torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _IO_TYPES.update({torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16, torch.int32: I32})
+        _TORCH = torch
+    return _TORCH
 
 
 def io_type(t) -> int:
-    torch = _torch()
-    if t.dtype == torch.float32:
-        return F32
-    if t.dtype == torch.bfloat16:
-        return BF16
-    if t.dtype == torch.float16:
-        return F16
-    if t.dtype == torch.int32:
-        return I32
-    raise DtError(f"unsupported dtype {t.dtype}")
+    _torch()
+    code = _IO_TYPES.get(t.dtype)
+    if code is None:
+        raise DtError(f"unsupported dtype {t.dtype}")
+    return code
+
+
+_I64x3 = c_int64 * 3
+
+
+@functools.lru_cache(maxsize=1024)
+def _i64x3(a, b, c):
+    return _I64x3(a, b, c)
+
+
+def _strides3(t):
+    a = t.stride()
+    return _i64x3(a[0], a[1], a[2])
 
 
 def _p(t):
@@ -266,7 +287,11 @@ def _p(t):
 
 
 def stream():
-    return c_void_p(_torch().cuda.current_stream().cuda_stream)
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return c_void_p(torch.cuda.current_stream().cuda_stream)
+    return c_void_p(raw(torch.cuda.current_device()))
 
 
 def desc(t, op=OP_NONE) -> DtTensor:
@@ -484,10 +509,21 @@ def quantize_q8_0(x, out=None):
     return y
 
 
+def _scratch(nbytes, device):
+    """Device scratch of one call: back in PyTorch's pool when the wrapper
+    returns, in stream order; prepare() keeps it for its repeats."""
+    torch = _torch()
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    lib = load()
+    if isinstance(lib, _Recorder):
+        lib.keep.append(ws)
+    return ws
+
+
 def _gemm_ws(nbytes, M, N, K, a):
     """Scratch for a product taken over ranges of K, or None for one that is not split."""
     n = nbytes(M, N, K)
-    return _torch().empty(n, dtype=_torch().uint8, device=a.device) if n else None
+    return _scratch(n, a.device) if n else None
 
 
 def gemm(a, b, bias=None, addend=None, out=None, out_dtype=None, config=-1):
@@ -506,7 +542,7 @@ def gemm(a, b, bias=None, addend=None, out=None, out_dtype=None, config=-1):
     if ws is not None:
         p = GemmProblem(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), out.data_ptr(), out.stride(0),
                         _p(addend), ldd, _p(bias), M, N, K, None, 0)
-        check(load().dt_gemm_bf16_ws(ctypes.byref(p), io_type(out), _p(ws), ws.numel(), stream()), "dt_gemm_bf16_ws")
+        check(load().dt_gemm_bf16_ws(ctypes.cast(ctypes.pointer(p), c_void_p), io_type(out), _p(ws), ws.numel(), stream()), "dt_gemm_bf16_ws")
         return out
     check(load().dt_gemm_bf16_config(_p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0),
                                      M, N, K, _p(bias), _p(addend), ldd, io_type(out), config,
@@ -554,7 +590,7 @@ def gemm_q8_0(a, w, bias=None, addend=None, out=None, out_dtype=None):
     if ws is not None:
         p = GemmProblem(a.data_ptr(), a.stride(0), w.codes.data_ptr(), w.codes.stride(0), out.data_ptr(),
                         out.stride(0), _p(addend), ldd, _p(bias), M, N, K, w.scales.data_ptr(), w.scales.stride(0))
-        check(load().dt_gemm_bf16_ws(ctypes.byref(p), io_type(out), _p(ws), ws.numel(), stream()), "dt_gemm_q8_0")
+        check(load().dt_gemm_bf16_ws(ctypes.cast(ctypes.pointer(p), c_void_p), io_type(out), _p(ws), ws.numel(), stream()), "dt_gemm_q8_0")
         return out
     check(load().dt_gemm_q8_0(_p(a), a.stride(0), _p(w.codes), w.codes.stride(0), _p(w.scales),
                               w.scales.stride(0), _p(out), out.stride(0), M, N, K, _p(bias), _p(addend), ldd,
@@ -605,7 +641,7 @@ def _conv_ws(x, workspace):
     torch = _torch()
     if workspace is True:
         N, ci, H, W = x.shape
-        return torch.empty(load().dt_conv2d_workspace_bytes(N, ci, H, W), dtype=torch.uint8, device=x.device)
+        return _scratch(load().dt_conv2d_workspace_bytes(N, ci, H, W), x.device)
     return workspace
 
 
@@ -659,7 +695,7 @@ def flash_attn(q, k, v, scale=None, out=None, out_dtype=None):
     Skv = k.shape[1]
     if out is None:
         out = torch.empty((B, Sq, H, D), dtype=out_dtype or torch.bfloat16, device=q.device)
-    st = lambda t: (c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
+    st = _strides3
     scale = 1.0 / D ** 0.5 if scale is None else scale
     check(load().dt_flash_attn_bf16(_p(q), _p(k), _p(v), _p(out), B, H, Sq, Skv, D, st(q), st(k),
                                     st(v), st(out), scale, io_type(out), stream()),
@@ -680,7 +716,7 @@ def gemm_f32(a, b, bias=None, addend=None, out=None):
     if ws is not None:
         p = GemmProblem(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), out.data_ptr(), out.stride(0),
                         _p(addend), ldd, _p(bias), M, N, K, None, 0)
-        check(load().dt_gemm_f32_ws(ctypes.byref(p), _p(ws), ws.numel(), stream()), "dt_gemm_f32")
+        check(load().dt_gemm_f32_ws(ctypes.cast(ctypes.pointer(p), c_void_p), _p(ws), ws.numel(), stream()), "dt_gemm_f32")
         return out
     check(load().dt_gemm_f32(_p(a), a.stride(0), _p(b), b.stride(0), _p(out), out.stride(0), M, N, K, _p(bias),
                              _p(addend), ldd, stream()), "dt_gemm_f32")
@@ -695,11 +731,11 @@ def flash_attn_f32(q, k, v, scale=None, out=None):
     Skv = k.shape[1]
     if out is None:
         out = torch.empty((B, Sq, H, D), dtype=torch.float32, device=q.device)
-    st = lambda t: (c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
+    st = _strides3
     scale = 1.0 / D ** 0.5 if scale is None else scale
     lib = load()
     nbytes = lib.dt_flash_attn_f32_workspace_bytes(B, H, Sq, Skv, D)
-    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=q.device)
+    ws = _scratch(max(nbytes, 16), q.device)
     check(lib.dt_flash_attn_f32(_p(q), _p(k), _p(v), _p(out), B, H, Sq, Skv, D, st(q), st(k), st(v), st(out),
                                 scale, _p(ws), ws.numel(), stream()), "dt_flash_attn_f32")
     return out
@@ -719,7 +755,7 @@ def flash_attn_qk(q_segments, k, v, pos, axis_dim, freq_base, eps=1e-6, table=No
     Skv = k.shape[1]
     if out is None:
         out = torch.empty((B, Sq, H, D), dtype=out_dtype or torch.bfloat16, device=k.device)
-    st = lambda t: (c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
+    st = _strides3
     scale = 1.0 / D ** 0.5 if scale is None else scale
     n_pos = 0 if table is None else table.shape[0]
     check(load().dt_flash_attn_qk_bf16(

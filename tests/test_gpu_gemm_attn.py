@@ -314,6 +314,22 @@ def test_gemm_few_tiles(orc, dev, M, N, K, weights, out_dtype):
     check(host(out2), lin, out_dtype, f"few tiles grouped {M}x{N}x{K}")
 
 
+def test_prepared_launch_keeps_its_scratch(orc, dev):
+    """prepare()'s repeats of calls with scratch of their own (K ranges of a
+    product, fp32 attention's parts) after that memory could be given away."""
+    a, b = dev_tensor(orc.randn(SEED + 274, (130, 576)), torch.bfloat16), dev_tensor(orc.randn(SEED + 275, (2050, 576)), torch.bfloat16)
+    q = dev_tensor(orc.randn(SEED + 276, (1, 70, 2, 128)), torch.float32)
+    for fn, args in ((dit_hip.gemm, (a, b)), (dit_hip.gemm_f32, (a.float(), b.float())), (dit_hip.flash_attn_f32, (q, q, q))):
+        out, launch = dit_hip.prepare(fn, *args)
+        first = out.clone()
+        others = [torch.full((n << 20,), 255, dtype=torch.uint8, device="cuda") for n in (1, 2, 4, 8, 16)]
+        out.zero_()
+        launch()
+        torch.cuda.synchronize()
+        assert torch.equal(out, first), fn.__name__
+        assert all((t == 255).all() for t in others), fn.__name__
+
+
 # ---------------------------------------------------------------- attention --
 def _attn_ref(orc, q, k, v, scale=None):
     """q [B, Sq, H, D] -> oracle attention per batch on the bf16-rounded values."""
