@@ -861,8 +861,32 @@ __global__ __launch_bounds__(512, 4) void conv1x1_kernel(const ConvArgs a, int64
         xofs[i] = trow * kPwPx * 2 + ((pair ^ (trow & 3)) << 5) + 8 * (s16 & 3);
     }
     const int wsw = ((lrow >> 1) ^ (lrow >> 2)) & 3;
-    auto tr = [](const uint8_t* p) {
-        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_p)(p)));
+    const uint32_t xlds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+    // Both 16-channel steps' pixel operands of one stage.  The wait is in the
+    // block; the compiler's own wait before its transposed reads would also drain the stage
+    // in flight (53 instead of 60 us at [1, 256, 512, 512] -> 128, profiled).
+    auto read_x = [&](int stage, bf16x8_t (&xf)[2][FN]) {
+        const uint32_t p0 = xlds + stage * kPwStage + xofs[0], p1 = xlds + stage * kPwStage + xofs[1];
+        uint2 r[8];
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %8\n\t"
+            "ds_read_b64_tr_b16 %1, %8 offset:2048\n\t"
+            "ds_read_b64_tr_b16 %2, %9\n\t"
+            "ds_read_b64_tr_b16 %3, %9 offset:2048\n\t"
+            "ds_read_b64_tr_b16 %4, %8 offset:8192\n\t"
+            "ds_read_b64_tr_b16 %5, %8 offset:10240\n\t"
+            "ds_read_b64_tr_b16 %6, %9 offset:8192\n\t"
+            "ds_read_b64_tr_b16 %7, %9 offset:10240\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+            : "v"(p0), "v"(p1)
+            : "memory");
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int i = 0; i < FN; ++i)
+                xf[kk][i] = __builtin_bit_cast(bf16x8_t, make_uint4(r[4 * kk + 2 * i].x, r[4 * kk + 2 * i].y,
+                                                                    r[4 * kk + 2 * i + 1].x, r[4 * kk + 2 * i + 1].y));
     };
     const int nch = a.Ci / kPwCi;
     issue(0, 0);
@@ -874,26 +898,21 @@ __global__ __launch_bounds__(512, 4) void conv1x1_kernel(const ConvArgs a, int64
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the stage refilled next
         __builtin_amdgcn_s_barrier();
         if (ch + 2 < nch) issue(ch + 2, st == 0 ? 2 : st - 1);
-        const uint8_t* X = smem + st * kPwStage;
-        const uint8_t* W = X + kPwX;
+        const uint8_t* W = smem + st * kPwStage + kPwX;
+        bf16x8_t wf[2][2], xf[2][FN];
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            bf16x8_t wf[2], xf[FN];
+        for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                wf[j] = *reinterpret_cast<const bf16x8_t*>(W + (wco + 32 * j + lrow) * 64 + (((2 * kk + g) ^ wsw) << 4));
+                wf[kk][j] = *reinterpret_cast<const bf16x8_t*>(W + (wco + 32 * j + lrow) * 64 + (((2 * kk + g) ^ wsw) << 4));
+        read_x(st, xf);
 #pragma unroll
-            for (int i = 0; i < FN; ++i) {
-                const uint2 lo = tr(X + xofs[i] + 16 * kk * kPwPx * 2);
-                const uint2 hi = tr(X + xofs[i] + (16 * kk + 4) * kPwPx * 2);
-                xf[i] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
-            }
+        for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int i = 0; i < FN; ++i)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], xf[i], acc[j][i], 0, 0, 0);
-        }
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk][j], xf[kk][i], acc[j][i], 0, 0, 0);
         st = st == kPwStages - 1 ? 0 : st + 1;
     }
     __syncthreads();  // the epilogue reuses the stages
