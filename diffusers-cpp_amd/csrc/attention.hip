@@ -403,7 +403,11 @@ __global__ __launch_bounds__(256, 2) void flash_attn_dma_kernel(AttnArgs a, Attn
 // K and V buffers of its own (8 KB each): a wave waits only for its own DMA and there
 // is no barrier until the four partial results meet in LDS.  K of the wave's next
 // tile loads from the end of its scores on, V from the end of P V on.  The
-// products, the softmax and its moving reference are flash_attn_dma_kernel's.
+// products, the softmax and its moving reference are flash_attn_dma_kernel's: every
+// wave starts from the largest score of keys 0-63, so P is rounded to bf16 at the
+// scale that kernel rounds it at (waves starting from their own first tile's differed from
+// it by 2.7e-3 in the 2-norm, all of it that rounding).  A reference that
+// is still -inf (every score so far -inf) gives its keys weight 0, not exp2(-inf + inf).
 // Kernel time (launches in one HIP graph), against blocks of 128: 24 heads of 320 16.1
 // -> 8.9 us, of 20 8.7 -> 6.0, 8 heads of 1000 28.8 -> 15.7, 2 of 2048 45 -> 23; past two
 // workgroups per CU K and V are read too often (24 heads of 700, 528 workgroups: 24.8
@@ -456,6 +460,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, Attn
     __shared__ __attribute__((aligned(16))) uint8_t smem[NW * 2 * FTILE];  // [wave][K | V]
     __shared__ __attribute__((aligned(16))) uint8_t qrows[PRO ? FTILE : 16];
     __shared__ float ml[2][NW][FQB];
+    __shared__ float first[2][FQB];  // per query: tile 0's and tile 1's largest scaled score
     uint32_t bid = blockIdx.x;
     const uint32_t nb = gridDim.x;
     if ((nb & 7u) == 0) bid = (bid & 7u) * (nb >> 3) + (bid >> 3);
@@ -525,6 +530,14 @@ __global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, Attn
         for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
     const float sc = a.scale_log2;
+    // Tile 0's and 1's maxima are in LDS.  Once per wave, whether or not it has a
+    // tile; not __syncthreads: the DMA stays in flight.
+    auto meet = [&]() {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's maxima are in LDS
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (wave >= ntiles) meet();
     for (int t = wave; t < ntiles; t += NW) {
         attn_wait_vm<8>();  // K (V's eight are younger)
         f32x16_t s[2];
@@ -549,6 +562,11 @@ __global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, Attn
             if (8 * (i >> 2) + 4 * g + (i & 3) < left) mx = fmaxf(mx, s[0][i]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 32));
+        if (t == wave) {
+            if (wave < 2 && g == 0) first[wave][r] = mx * sc;
+            meet();
+            m_run = ntiles > 1 ? fmaxf(first[0][r], first[1][r]) : first[0][r];
+        }
         const float m_cand = fmaxf(m_run, mx * sc);
         const bool move = m_cand > m_run + 8.0f;
         if (__builtin_amdgcn_ballot_w64(move)) {
@@ -561,6 +579,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, Attn
                 for (int e = 0; e < 16; ++e) o[tt][e] *= alpha;
             m_run = m_new;
         }
+        const float m_sub = m_run == -INFINITY ? 0.f : m_run;
         float psum = 0.f;
         bf16x8_t pf[2];
 #pragma unroll
@@ -572,7 +591,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, Attn
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
                     const int i = 8 * j + e + u;
-                    float arg = __builtin_fmaf(s[0][i], sc, -m_run);
+                    float arg = __builtin_fmaf(s[0][i], sc, -m_sub);
                     if (8 * (i >> 2) + 4 * g + (i & 3) >= left) arg = -INFINITY;
                     p2[u] = __builtin_amdgcn_exp2f(arg);
                     psum += p2[u];

@@ -651,3 +651,51 @@ def test_flash_attn_qk_prologue_rejects(dev):
         dit_hip.flash_attn_qk([(z, w)], z, z, pos, 24, 10000.0)      # 4 x 24 != 128
     with pytest.raises(dit_hip.DtError, match="axis_dim"):
         dit_hip.flash_attn_qk([(z, w)], z, z, pos[:, :2], 36, 10000.0)  # axis_dim % 8 != 0
+@pytest.mark.parametrize("lo,hi", [(32, 64), (0, 32), (0, 64), (64, 96), (96, 200)])
+@pytest.mark.parametrize("inf", [True, False])
+def test_flash_attn_minus_inf_tiles(dev, lo, hi, inf):
+    """Keys [lo, hi) whose scores are all -inf (infinite K, or finite operands
+    whose sum overflows), in blocks of 32 queries: weight 0, as with every key
+    tile that a wave does not begin on; all keys -inf gives NaN."""
+    print(f"attn -inf keys {lo}..{hi} inf={inf}", flush=True)
+    g = torch.Generator().manual_seed(SEED + 251)
+    q = torch.rand((1, 40, 2, 128), generator=g) + 0.5
+    k, v = torch.randn((1, 200, 2, 128), generator=g) * 0.1, torch.randn((1, 200, 2, 128), generator=g)
+    dead = (Ellipsis,) if inf else (0,)  # the dims that make a score -inf
+    if not inf:
+        q[:, :, 0, 0], k[:, :, 0, 0] = 0.0, 0.0
+        q[:, 3, 0, 0] = 1e20
+    k[(0, slice(lo, hi), 0) + dead] = float("-inf") if inf else -1e20
+    qd, kd, vd = (t.bfloat16().cuda() for t in (q, k, v))
+    o = dit_hip.flash_attn(qd, kd, vd).float().cpu()
+    k[(0, slice(None), 0) + dead] = float("-inf") if inf else -1e20
+    none = dit_hip.flash_attn(qd, k.bfloat16().cuda(), vd).float().cpu()
+    torch.cuda.synchronize()
+    rows = slice(None) if inf else slice(3, 4)
+    assert torch.isnan(none[:, rows, 0]).all() and not torch.isnan(none[:, :, 1]).any()
+    qf, kf, vf = (t.float().cpu().permute(0, 2, 1, 3) for t in (qd, kd, vd))
+    s = (qf @ kf.transpose(-1, -2).contiguous()) / 128 ** 0.5
+    ref = (torch.softmax(s.double(), -1) @ vf.double()).permute(0, 2, 1, 3)
+    assert not torch.isnan(o).any()
+    assert_bf16(o.numpy(), ref.float().numpy(), f"attention with keys {lo}..{hi} at -inf")
+
+
+@pytest.mark.parametrize("Sq,Skv,H", [(320, 320, 24), (40, 33, 2), (33, 500, 3), (20, 1000, 5)])
+def test_flash_attn_block_sizes_agree(dev, Sq, Skv, H):
+    """Blocks of 32 queries and (the same inputs in a batch too large for them) of
+    128: softmax weights rounded to bf16 at the same scale, so what differs is the
+    order of fp32 sums.  That moves an exponent by about 2^-21 and so 2^-21 / 2^-9
+    of the weights and results across a bf16 rounding step of 2^-8: sqrt(2^-12)
+    2^-8 = 6e-5 in the 2-norm, four times which is allowed.  (Weights rounded at scales
+    of their own differ by 2.7e-3.)"""
+    print(f"attn block sizes agree Sq={Sq} Skv={Skv} H={H}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(SEED + 252)
+    q, k, v = (torch.randn((1, S, H, 128), generator=g, device="cuda").bfloat16() for S in (Sq, Skv, Skv))
+    few = dit_hip.flash_attn(q, k, v)
+    B = 1024 // (H * ((Sq + 31) // 32)) + 1  # over two blocks of 32 queries per CU
+    many = dit_hip.flash_attn(*(t.expand(B, -1, -1, -1).contiguous() for t in (q, k, v)))
+    torch.cuda.synchronize()
+    a, b = few[0].double(), many[B // 2].double()
+    assert ((a - b).norm() / b.norm()).item() <= 2.4e-4
+
+
