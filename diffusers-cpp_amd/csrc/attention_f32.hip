@@ -32,8 +32,10 @@
 // P V run, V of the next tile while its scores are computed.
 //
 // A (batch, head) with operands outside the range in which the parts are normal
-// numbers (|q|, |k| >= 2^50, |v| >= 2^30 or 0 < |v| < 2^-60, not finite) is taken in
-// plain fp32 arithmetic instead (attn_plain).
+// numbers (|q|, |k| >= 2^50, |v| >= 2^30 or 0 < |v| < 2^-60, not finite) is taken on
+// the fp32 matrix cores instead (attn_native): 24 heads of 1536 x 1536 with one such element a head
+// 840 us, 8 of 1000 326, 24 of 320 176 (a query at a time by hand 18.7 ms, 6.1 and 2.4; through GEMMs
+// 1112, 318 and 347 us).
 #include <math.h>
 
 #include <initializer_list>
@@ -125,66 +127,131 @@ __global__ __launch_bounds__(256) void split_kv_kernel(const F32Attn a) {
     if (threadIdx.x == 0) a.flags[((int64_t)bh * 2 + blockIdx.z) * a.kv_blocks + blockIdx.x] = any ? 1u : 0u;
 }
 
-// Queries [q0, q0 + QB) of one head in fp32 arithmetic, one at a time: a thread per
-// key of a 256-key tile for the scores, a thread per d for O.
-__device__ void attn_plain(const F32Attn& a, int b, int h, int q0, float* lds) {
-    float* qrow = lds;           // [128]
-    float* p = lds + D;          // [256]
-    float* red = lds + D + 256;  // [4] per-wave results
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// Queries [q0, q0 + QB) of one head on the fp32 matrix cores
+// (v_mfma_f32_32x32x2_f32), for operands of any magnitude: the arithmetic of the
+// GEMM path (gemm_f32.hip) tile by tile.  The keys are walked twice, for
+// each query's largest score m and l = sum expf(scale s - m), then for O = sum
+// (expf(scale s - m) / l) v, so no product exceeds the largest |v|.  A row whose scores are
+// -inf so far keeps the weights 0; rows with a NaN or +inf score, or none above -inf, are NaN.
+// K and V tiles of 32 keys pass through LDS, the next one on its way in registers.  As in the
+// kernel below lane l holds query l % 32 and, of a 32 x 32 block, key (or d) 8 (i / 4) +
+// 4 (l / 32) + i % 4; MFMA step 4 c + e of the scores takes d = 8 c + 4 (l / 32) + e, step i
+// of P V the keys of score element i, so P goes from one to the other in place.
+__device__ void attn_native(const F32Attn& a, int b, int h, int q0, float* lds) {
+    constexpr int LD = D + 4;  // padded row: 16 rows' 16-byte reads hit distinct banks
+    float* const Kt = lds;
+    float* const Vt = lds + KB * LD;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, g = lane >> 5, q = q0 + 32 * wave + r;
     const float* kb = a.k + b * a.ks[0] + h * a.ks[2];
     const float* vb = a.v + b * a.vs[0] + h * a.vs[2];
-    for (int q = q0; q < min(q0 + QB, a.seq_q); ++q) {
-        __syncthreads();
-        if (tid < D) qrow[tid] = a.q[b * a.qs[0] + q * a.qs[1] + h * a.qs[2] + tid];
-        __syncthreads();
-        float m = -INFINITY, l = 0.f, o = 0.f;
-        for (int k0 = 0; k0 < a.seq_kv; k0 += 256) {
-            const int key = k0 + tid;
-            float s = -INFINITY;
-            if (key < a.seq_kv) {
-                float part[4] = {0.f, 0.f, 0.f, 0.f};
-                for (int d = 0; d < D; d += 4)
+    // Q is read again for every tile: 64 registers more would spill.
+    const float* qp = a.q + b * a.qs[0] + (int64_t)min(q, a.seq_q - 1) * a.qs[1] + h * a.qs[2] + 4 * g;
+
+    // Thread t: float4 t % 32 of rows t / 32 + 8 u; zeros past seq_kv (a masked weight
+    // must not meet a NaN).
+    const int srow = tid >> 5, scol = 4 * (tid & 31);
+    auto fetch = [&](const float* src, int64_t ts, int k0, float4 (&x)[4]) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        part[e] = __builtin_fmaf(qrow[d + e], kb[key * a.ks[1] + d + e], part[e]);
-                s = a.scale * ((part[0] + part[1]) + (part[2] + part[3]));
-            }
-            // A NaN score makes the row NaN, as a sum over it would.
-            float mx = s, bad = s != s ? 1.f : 0.f;
-            for (int off = 32; off > 0; off >>= 1) {
-                mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-                bad = fmaxf(bad, __shfl_xor(bad, off, kWave));
-            }
-            if (lane == 0) red[wave] = bad != 0.f ? NAN : mx;
-            __syncthreads();
-            float mt = m;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) mt = red[w] != red[w] || mt != mt ? NAN : fmaxf(mt, red[w]);
-            const float pv = key < a.seq_kv ? expf(s - mt) : 0.f;
-            p[tid] = pv;
-            const float ws = wave_sum(pv);
-            __syncthreads();
-            if (lane == 0) red[wave] = ws;
-            __syncthreads();
-            const float alpha = expf(m - mt);
-            l = l * alpha + ((red[0] + red[1]) + (red[2] + red[3]));
-            m = mt;
-            if (tid < D) {
-                float part[4] = {0.f, 0.f, 0.f, 0.f};
-                const int n = min(256, a.seq_kv - k0);
-                int j = 0;
-                for (; j + 4 <= n; j += 4)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        part[e] = __builtin_fmaf(p[j + e], vb[(int64_t)(k0 + j + e) * a.vs[1] + tid], part[e]);
-                for (; j < n; ++j) part[0] = __builtin_fmaf(p[j], vb[(int64_t)(k0 + j) * a.vs[1] + tid], part[0]);
-                o = o * alpha + ((part[0] + part[1]) + (part[2] + part[3]));
-            }
-            __syncthreads();
+        for (int u = 0; u < 4; ++u) {
+            const int key = k0 + srow + 8 * u;
+            x[u] = key < a.seq_kv ? *reinterpret_cast<const float4*>(src + key * ts + scol) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        if (tid < D) a.o[b * a.os[0] + q * a.os[1] + h * a.os[2] + tid] = o / l;
+    };
+    auto stash = [&](float* dst, const float4 (&x)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<float4*>(dst + (srow + 8 * u) * LD + scol) = x[u];
+    };
+    // scale s of the K tile from key k0, -inf past seq_kv; two running sums.
+    auto scores = [&](int k0, float (&s)[16]) {
+        f32x16_t acc[2];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[0][e] = acc[1][e] = 0.f;
+#pragma unroll 4
+        for (int c = 0; c < 16; ++c) {
+            const float4 kv = *reinterpret_cast<const float4*>(Kt + r * LD + 8 * c + 4 * g);
+            const float4 qv = *reinterpret_cast<const float4*>(qp + 8 * c);
+            const float kx[4] = {kv.x, kv.y, kv.z, kv.w}, qx[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                acc[e & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[e], qx[e], acc[e & 1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = a.scale * (acc[0][i] + acc[1][i]);
+            if (k0 + 8 * (i >> 2) + 4 * g + (i & 3) >= a.seq_kv) s[i] = -INFINITY;
+        }
+    };
+
+    float m = -INFINITY, l = 0.f, l_err = 0.f;
+    float4 nk[4], nv[4];
+    fetch(kb, a.ks[1], 0, nk);
+    for (int k0 = 0; k0 < a.seq_kv; k0 += KB) {
+        __syncthreads();  // every wave has read the tile before
+        stash(Kt, nk);
+        __syncthreads();
+        if (k0 + KB < a.seq_kv) fetch(kb, a.ks[1], k0 + KB, nk);
+        float s[16], mt = m;
+        scores(k0, s);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mt = fmaxf(mt, s[i]);
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        const float ref = mt == -INFINITY ? 0.f : mt, alpha = expf(m - ref);
+        float ts = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ts += expf(s[i] - ref);
+        m = mt;
+        l *= alpha;
+        l_err *= alpha;
+        const float n = l + ts, bb = n - l;  // l + l_err += ts
+        l_err += (l - (n - bb)) + (ts - bb);
+        l = n;
     }
+    l += l_err;
+    const float inv = 1.0f / (l + __shfl_xor(l, 32)), ref = m == -INFINITY ? 0.f : m;
+
+    f32x16_t o[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
+    fetch(kb, a.ks[1], 0, nk);
+    for (int k0 = 0; k0 < a.seq_kv; k0 += KB) {
+        __syncthreads();
+        stash(Kt, nk);
+        __syncthreads();
+        fetch(vb, a.vs[1], k0, nv);
+        float p[16];
+        scores(k0, p);
+        stash(Vt, nv);
+        __syncthreads();
+        if (k0 + KB < a.seq_kv) fetch(kb, a.ks[1], k0 + KB, nk);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            p[i] = expf(p[i] - ref) * inv;
+            if (k0 + 8 * (i >> 2) + 4 * g + (i & 3) >= a.seq_kv) p[i] = 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x16_t acc;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Vt[(8 * (i >> 2) + 4 * g + (i & 3)) * LD + 32 * t + r], p[i], acc,
+                                                           0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[t][e] += acc[e];
+        }
+    }
+    if (q >= a.seq_q) return;
+    float* op = a.o + b * a.os[0] + (int64_t)q * a.os[1] + h * a.os[2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+            *reinterpret_cast<float4*>(op + 32 * t + 8 * i4 + 4 * g) =
+                make_float4(o[t][4 * i4], o[t][4 * i4 + 1], o[t][4 * i4 + 2], o[t][4 * i4 + 3]);
 }
 
 __device__ __forceinline__ uint2 read_tr16(const uint8_t* p) {
@@ -241,7 +308,8 @@ __global__ __launch_bounds__(256, 2) void flash_attn_f32_kernel(const F32Attn a)
         // attn_combine_kernel leaves rows with l = NaN as they are
         if (a.splits > 1 && q < a.seq_q && g == 0)
             a.ml[((int64_t)split * a.bh + bh) * a.seq_q + q] = make_float2(0.f, NAN);
-        if (split == 0) attn_plain(a, b, h, qblk * QB, reinterpret_cast<float*>(smem));
+        static_assert(2 * KB * (D + 4) * (int)sizeof(float) <= 2 * TILEB, "attn_native's tiles");
+        if (split == 0) attn_native(a, b, h, qblk * QB, reinterpret_cast<float*>(smem));
         return;
     }
 

@@ -485,6 +485,53 @@ def test_flash_attn_f32_ranges(dev, B, Sq, Skv, H, case):
     assert ((got - ref).abs()[ok] <= max(1e-5, 2.0 ** -23 * smax) * vmax[ok]).all()
 
 
+@pytest.mark.parametrize("case", ["inf_keys", "overflow", "uniform_huge_v", "late_max", "nan_row", "ragged_inf"])
+def test_flash_attn_f32_native(dev, case):
+    """Heads taken on the fp32 matrix cores: scores of -inf over the first 256
+    keys (infinite K; finite operands whose sum overflows), weights near 1 / Skv
+    on |v| near the largest float, a maximum in the last tile, NaN rows, and
+    infinities in the last (partial) key tile and query block."""
+    print(f"attn_f32 native {case}", flush=True)
+    g = torch.Generator().manual_seed(SEED + 293)
+    Sq, Skv, H, far = 140, 301, 2, 256
+    q, k, v = torch.rand((1, Sq, H, 128), generator=g) + 0.5, *(torch.randn((1, Skv, H, 128), generator=g) for _ in "kv")
+    dead = torch.zeros((Sq, Skv), dtype=torch.bool)  # head 0's scores that are -inf
+    if case == "inf_keys":
+        k[:, :far, 0], dead[:, :far] = float("-inf"), True
+    elif case == "overflow":
+        q[:, 1::2, 0] = 2.0 ** 64
+        k[:, :far, 0] = -2.0 ** 64
+        k[:, far:, 0] = torch.arange(Skv - far).float()[None, :, None]
+        dead[:, :far] = True
+    elif case == "uniform_huge_v":
+        q[:, :, 0], v[:, :, 0] = 0.0, 1e38 * torch.sign(v[:, :1, 0])
+    elif case == "late_max":
+        v[0, 0, 0, 0] = 2.0 ** -120  # out of range: head 0 is native
+        k[:, -1, 0] = 4.0
+    elif case == "nan_row":
+        q[0, 5, 0, 3] = float("nan")
+    else:
+        k[:, -1, 0], dead[:, -1] = float("-inf"), True
+        q[0, -1, 0, 0] = float("inf")
+    o = dit_hip.flash_attn_f32(*(t.cuda() for t in (q, k, v))).cpu().double()
+    torch.cuda.synchronize()
+    qd, kd, vd = (t[0].double().permute(1, 0, 2) for t in (q, k, v))
+    s = qd @ kd.transpose(-1, -2).contiguous() / 128 ** 0.5
+    s[0][dead] = float("-inf")
+    if case == "ragged_inf":
+        s[0, -1] = float("nan")  # inf against keys of both signs
+    ref = torch.softmax(s, -1) @ vd
+    got = o[0].permute(1, 0, 2)
+    nan = torch.isnan(ref)
+    assert torch.equal(torch.isnan(got), nan), case
+    # a score's fp32 rounding, 2^-24 of 128 products' magnitudes, moves a weight by as much
+    live = torch.where(torch.isfinite(s), s.abs(), 0.0).amax(-1, keepdim=True)
+    if case == "overflow":
+        live = live.clamp(max=64.0)  # one key's weight is 1: its score moves nothing
+    bound = (1e-5 + 2.0 ** -22 * live) * vd.abs().amax((1, 2), keepdim=True)
+    assert ((got - ref).abs() <= bound)[~nan].all(), case
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,Sq,Skv,H", ATTN_SHAPES)
 def test_flash_attn(orc, dev, B, Sq, Skv, H, out_dtype):
@@ -651,6 +698,8 @@ def test_flash_attn_qk_prologue_rejects(dev):
         dit_hip.flash_attn_qk([(z, w)], z, z, pos, 24, 10000.0)      # 4 x 24 != 128
     with pytest.raises(dit_hip.DtError, match="axis_dim"):
         dit_hip.flash_attn_qk([(z, w)], z, z, pos[:, :2], 36, 10000.0)  # axis_dim % 8 != 0
+
+
 @pytest.mark.parametrize("lo,hi", [(32, 64), (0, 32), (0, 64), (64, 96), (96, 200)])
 @pytest.mark.parametrize("inf", [True, False])
 def test_flash_attn_minus_inf_tiles(dev, lo, hi, inf):
@@ -697,5 +746,3 @@ def test_flash_attn_block_sizes_agree(dev, Sq, Skv, H):
     torch.cuda.synchronize()
     a, b = few[0].double(), many[B // 2].double()
     assert ((a - b).norm() / b.norm()).item() <= 2.4e-4
-
-
