@@ -32,7 +32,7 @@
 // P V run, V of the next tile while its scores are computed.
 //
 // A (batch, head) with operands outside the range in which the parts are normal
-// numbers (|q|, |k| >= 2^50, |v| >= 2^30 or 0 < |v| < 2^-60, not finite) is taken on
+// numbers (|q|, |k| >= 2^50, |v| >= 2^30 or 0 < |v| < 2^-80, not finite) is taken on
 // the fp32 matrix cores instead (attn_native): 24 heads of 1536 x 1536 with one such element a head
 // 840 us, 8 of 1000 326, 24 of 320 176 (a query at a time by hand 18.7 ms, 6.1 and 2.4; through GEMMs
 // 1112, 318 and 347 us).
@@ -58,7 +58,9 @@ constexpr int ROWB = 3 * D * 2, TILEB = KB * ROWB;
 constexpr int SPLIT_ROWS = 64;                // rows per workgroup of split_kv_kernel
 constexpr float kQkMax = 1125899906842624.0f;      // 2^50
 constexpr float kVMax = 1073741824.0f;             // 2^30
-constexpr float kVMin = 8.6736173798840355e-19f;   // 2^-60
+// A product of parts is lost below 2^-126, and a row's largest weight is at
+// least 1 before the division by l: n keys lose under 6 n 2^-46 of a result of this size.
+constexpr float kVMin = 8.2718061255302767e-25f;   // 2^-80
 
 struct F32Attn {
     const float* q;

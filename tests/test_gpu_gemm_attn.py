@@ -532,6 +532,26 @@ def test_flash_attn_f32_native(dev, case):
     assert ((got - ref).abs() <= bound)[~nan].all(), case
 
 
+@pytest.mark.parametrize("tiny", [2.0 ** -62, 2.0 ** -79])
+def test_flash_attn_f32_one_tiny_v(dev, tiny):
+    """One tiny element among ordinary V takes its head to no other arithmetic:
+    every other column is bit for bit what it is with a zero there, its own
+    within fp32's rounding."""
+    print(f"attn_f32 one tiny v {tiny}", flush=True)
+    g = torch.Generator().manual_seed(SEED + 294)
+    q, k, v = (torch.randn((1, S, 2, 128), generator=g).cuda() for S in (70, 130, 130))
+    v[0, :, 0, 5] = 0.0
+    zero = dit_hip.flash_attn_f32(q, k, v)
+    v[0, 9, 0, 5] = tiny
+    got = dit_hip.flash_attn_f32(q, k, v)
+    torch.cuda.synchronize()
+    col = got[0, :, 0, 5].double().clone()
+    p = torch.softmax((q[0, :, 0].double() @ k[0, :, 0].double().t().contiguous()) / 128 ** 0.5, -1)[:, 9] * tiny
+    assert ((col - p).abs() <= 1e-5 * tiny).all()
+    got[0, :, 0, 5] = 0.0
+    assert torch.equal(got, zero)
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,Sq,Skv,H", ATTN_SHAPES)
 def test_flash_attn(orc, dev, B, Sq, Skv, H, out_dtype):
