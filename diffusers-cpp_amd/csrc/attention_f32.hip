@@ -62,6 +62,8 @@ constexpr float kVMax = 1073741824.0f;             // 2^30
 // least 1 before the division by l: n keys lose under 6 n 2^-46 of a result of this size.
 constexpr float kVMin = 8.2718061255302767e-25f;   // 2^-80
 
+constexpr float kScaleMax = 1208925819614629174706176.0f;  // 2^80
+
 struct F32Attn {
     const float* q;
     const float* k;
@@ -545,7 +547,8 @@ size_t attn_f32_fused_bytes(int64_t batch, int64_t heads, int64_t seq_q, int64_t
 bool attn_f32_fused_takes(const float* q, const float* k, const float* v, const float* o, int64_t batch, int64_t heads,
                           int64_t seq_q, int64_t seq_kv, int64_t head_dim, const int64_t* qs, const int64_t* ks,
                           const int64_t* vs, const int64_t* os, float scale) {
-    if (head_dim != D || !(scale >= 0.f) || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
+    // Parts of a score lost below 2^-126 stay under 2^-38 after the scale.
+    if (head_dim != D || !(scale >= 0.f && scale <= kScaleMax) || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
         return false;
     for (int i = 0; i < 3; ++i)
         if (qs[i] % 4 || ks[i] % 4 || vs[i] % 4 || os[i] % 4) return false;

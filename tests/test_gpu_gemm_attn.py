@@ -552,6 +552,25 @@ def test_flash_attn_f32_one_tiny_v(dev, tiny):
     assert torch.equal(got, zero)
 
 
+@pytest.mark.parametrize("up", [79, 81, 127])
+def test_flash_attn_f32_large_scale(dev, up):
+    """q k around 2^-up with a scale of 1.75 2^up: on either side of the scale that
+    the split products are used for, and one whose log2(e) multiple is infinite."""
+    print(f"attn_f32 scale 1.75 2^{up}", flush=True)
+    g = torch.Generator().manual_seed(SEED + 295)
+    q, k, v = (torch.randn((1, S, 2, 128), generator=g) for S in (70, 130, 130))
+    q, k = q * 2.0 ** -(up // 2), k * 2.0 ** -(up - up // 2 + 3)
+    o = torch.full((1, 70, 2, 128), float("nan"), device="cuda")
+    dit_hip.flash_attn_f32(q.cuda(), k.cuda(), v.cuda(), scale=1.75 * 2.0 ** up, out=o)
+    torch.cuda.synchronize()
+    qd, kd, vd = (t[0].double().permute(1, 0, 2) for t in (q, k, v))
+    ref = torch.softmax(qd @ kd.transpose(-1, -2).contiguous() * (1.75 * 2.0 ** up), -1) @ vd
+    # 128 products of a score may each lose 2^-126 times the scale below fp32's range
+    bound = 1e-5 + 128 * 2.0 ** (up - 126)
+    got = o.cpu().double()[0].permute(1, 0, 2)
+    assert ((got - ref).abs() <= min(bound, 0.25) * vd.abs().max()).all(), (got - ref).abs().max().item()
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,Sq,Skv,H", ATTN_SHAPES)
 def test_flash_attn(orc, dev, B, Sq, Skv, H, out_dtype):
