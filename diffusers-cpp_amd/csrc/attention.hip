@@ -114,43 +114,87 @@ __device__ __forceinline__ uint2 read_tr16(const uint8_t* p) {
     return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_p)(p)));
 }
 
-// Chunk c (8 dims) of query q0 + row with QK-RMSNorm + RoPE applied, 16 lanes a
-// query, as bf16 into row `row` of `rows` in LDS (chunk c at c ^ (row & 15)).  Every
-// operation is the QK kernel's (qk_rope.hip), in its order: per 8-dim chunk the sum of
-// squares, the 16 chunk sums added by its 16-lane DPP tree, 1 / sqrt(ss / 128 +
-// eps), (x * r) * w, the rotation, one bf16 rounding -- so the q used here is
-// bit-identical to the stored output of dt_qk_rmsnorm_rope.  (A lane taking half of a
+// Chunk c (8 dims) of queries q0 + row, + row + 4, ... (N of them) with QK-RMSNorm + RoPE
+// applied, 16 lanes a query, as bf16 into their rows of `rows` in LDS (chunk c of row r at
+// c ^ (r & 15)).  Every operation is the QK kernel's (qk_rope.hip), in its order: per
+// 8-dim chunk the sum of squares, the 16 chunk sums added by its 16-lane DPP tree, 1 /
+// sqrt(ss / 128 + eps), (x * r) * w, the rotation, one bf16 rounding -- so the q used here
+// is bit-identical to the stored output of dt_qk_rmsnorm_rope.  (A lane taking half of a
 // query's chunks, as its MFMA operand holds them, made 16-byte loads of 64 scattered
 // lines and a long unrolled body: about 5 us of the 16.5 a 320-token attention took.)
+// All N queries' loads are issued before the first is used, and the angles' loads,
+// which wait for the positions, together: query by query each of a wave's eight waited
+// for memory twice.  With operands from HBM (many input sets in turn): 16 heads of 1068
+// 36.7 -> 33.4 us, 24 of 700 28.7 -> 25.3, 24 of 1536 56.5 -> 52.8, 24 of 320 10.1 -> 9.7.
+template <int N>
 __device__ __forceinline__ void q_prologue16(const AttnPro& pro, int b, int h, int q0, int row, int seq_q, int c,
                                              uint8_t* rows) {
-    const int qrow = min(q0 + row, seq_q - 1);  // rows past the sequence are never stored
-    const int seg = qrow >= pro.split, tok = seg ? qrow - pro.split : qrow;
-    const uint16_t* src = seg ? pro.q1 + b * pro.q1_bs + (int64_t)tok * pro.q1_ts + h * pro.q1_hs
-                              : pro.q0 + b * pro.q0_bs + (int64_t)tok * pro.q0_ts + h * pro.q0_hs;
-    const int d0 = 8 * c, axis = d0 / pro.axis_dim;
-    const int p = pro_position(pro.pos, axis, qrow);
-    const uint4 raw = ld16(src + d0);
-    const float* w = (seg ? pro.w1 : pro.w0) + d0;
-    const float4 wa = *reinterpret_cast<const float4*>(w), wb = *reinterpret_cast<const float4*>(w + 4);
-    const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
-    float cs[8], v[8], o[8];
-    rope_angles<4>(p, d0 - axis * pro.axis_dim, pro.table, pro.n_pos, pro.axis_dim, pro.theta_scale, cs);
-    Io<bf16>::unpack(raw, v);
-    float ss = 0.f;
+    const int d0 = 8 * c, axis = d0 / pro.axis_dim, i0 = d0 - axis * pro.axis_dim;
+    auto emit = [&](int n, const uint4& raw, const float (&cs)[8]) {
+        const float* w = (min(q0 + row + 4 * n, seq_q - 1) >= pro.split ? pro.w1 : pro.w0) + d0;
+        const float4 wa = *reinterpret_cast<const float4*>(w), wb = *reinterpret_cast<const float4*>(w + 4);
+        const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
+        float v[8], o[8];
+        Io<bf16>::unpack(raw, v);
+        float ss = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-    ss = row16_sum(ss);
-    const float rs = 1.0f / sqrtf(ss / (float)D + pro.eps);
+        for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+        ss = row16_sum(ss);
+        const float rs = 1.0f / sqrtf(ss / (float)D + pro.eps);
 #pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-        const float x0 = mul_rn(mul_rn(v[2 * qd], rs), wv[2 * qd]);
-        const float x1 = mul_rn(mul_rn(v[2 * qd + 1], rs), wv[2 * qd + 1]);
-        const float cn = cs[2 * qd], sn = cs[2 * qd + 1];
-        o[2 * qd] = sub_rn(mul_rn(x0, cn), mul_rn(x1, sn));
-        o[2 * qd + 1] = add_rn(mul_rn(x0, sn), mul_rn(x1, cn));
+        for (int qd = 0; qd < 4; ++qd) {
+            const float x0 = mul_rn(mul_rn(v[2 * qd], rs), wv[2 * qd]);
+            const float x1 = mul_rn(mul_rn(v[2 * qd + 1], rs), wv[2 * qd + 1]);
+            const float cn = cs[2 * qd], sn = cs[2 * qd + 1];
+            o[2 * qd] = sub_rn(mul_rn(x0, cn), mul_rn(x1, sn));
+            o[2 * qd + 1] = add_rn(mul_rn(x0, sn), mul_rn(x1, cn));
+        }
+        const int r = row + 4 * n;
+        *reinterpret_cast<uint4*>(rows + r * DROW + ((c ^ (r & 15)) << 4)) = Io<bf16>::pack(o);
+    };
+    int p[N];
+    uint4 raw[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const int qrow = min(q0 + row + 4 * n, seq_q - 1);  // rows past the sequence are never stored
+        const int seg = qrow >= pro.split, tok = seg ? qrow - pro.split : qrow;
+        p[n] = pro_position(pro.pos, axis, qrow);
+        raw[n] = ld16((seg ? pro.q1 + b * pro.q1_bs + (int64_t)tok * pro.q1_ts + h * pro.q1_hs
+                           : pro.q0 + b * pro.q0_bs + (int64_t)tok * pro.q0_ts + h * pro.q0_hs) + d0);
     }
-    *reinterpret_cast<uint4*>(rows + row * DROW + ((c ^ (row & 15)) << 4)) = Io<bf16>::pack(o);
+    bool hit = pro.table != nullptr;
+#pragma unroll
+    for (int n = 0; n < N; ++n) hit = hit && p[n] >= 0 && p[n] < pro.n_pos;
+    if (__builtin_amdgcn_ballot_w64(!hit) == 0) {  // every angle from the table
+        float cs[N][8];
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const float* t = pro.table + (int64_t)p[n] * pro.axis_dim + i0;  // rope_angles' table branch
+            const float4 ca = *reinterpret_cast<const float4*>(t), cb = *reinterpret_cast<const float4*>(t + 4);
+            cs[n][0] = ca.x; cs[n][1] = ca.y; cs[n][2] = ca.z; cs[n][3] = ca.w;
+            cs[n][4] = cb.x; cs[n][5] = cb.y; cs[n][6] = cb.z; cs[n][7] = cb.w;
+        }
+#pragma unroll
+        for (int n = 0; n < N; ++n) emit(n, raw[n], cs[n]);
+    } else {
+        // Some angle off the table: unrolled for eight queries this body would
+        // put their registers into scratch memory.
+        constexpr int U = N <= 2 ? N : 1;
+#pragma unroll U
+        for (int n = 0; n < N; ++n) {
+            int pn = p[0];
+            uint4 rn = raw[0];
+#pragma unroll
+            for (int i = 1; i < N; ++i)
+                if (n == i) {
+                    pn = p[i];
+                    rn = raw[i];
+                }
+            float cs[8];
+            rope_angles<4>(pn, i0, pro.table, pro.n_pos, pro.axis_dim, pro.theta_scale, cs);
+            emit(n, rn, cs);
+        }
+    }
 }
 
 template <typename TO, bool PRO>
@@ -350,9 +394,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_dma_kernel(AttnArgs a, Attn
         // 32) x 256 B.  Every wave has read its rows back before the
         // barrier, and the buffer's first DMA comes after it.
         uint8_t* rows = smem + 2 * DTILE + 32 * wave * DROW;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            q_prologue16(pro, b, h, q0, 4 * i + (lane >> 4), a.seq_q, lane & 15, rows);
+        q_prologue16<8>(pro, b, h, q0, lane >> 4, a.seq_q, lane & 15, rows);
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's rows are in LDS
 #pragma unroll
         for (int c = 0; c < 8; ++c)
@@ -493,9 +535,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_few_kernel(AttnArgs a, Attn
     // Each wave prepares eight of the block's queries for all.
     bf16x8_t qf[8];
     if constexpr (PRO) {
-#pragma unroll
-        for (int i = 0; i < FQB / (4 * NW); ++i)
-            q_prologue16(pro, b, h, qblk * FQB, (FQB / NW) * wave + 4 * i + (lane >> 4), a.seq_q, lane & 15, qrows);
+        q_prologue16<FQB / (4 * NW)>(pro, b, h, qblk * FQB, (FQB / NW) * wave + (lane >> 4), a.seq_q, lane & 15, qrows);
         // Not __syncthreads: K's DMA stays in flight.
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's rows are in LDS
         __builtin_amdgcn_s_barrier();
