@@ -1112,6 +1112,23 @@ int64_t tiles_of(const Problem& p, int cfg) {
     return (int64_t)((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
 }
 
+// Whether configuration cfg can address every problem's tiles: gemm_k64_kernel's
+// buffer loads reach 2^31 bytes from a tile's first row (gemm_128_kernel, config 1,
+// has 64-bit row offsets).
+bool reaches(const Problem* ps, int n, int cfg) {
+    if (cfg == 1) return true;
+    constexpr int64_t kReach = 0x7FFFFFFF;
+    for (int i = 0; i < n; ++i) {
+        const Problem& p = ps[i];
+        const int64_t ra = (p.M < kConfigs[cfg].bm ? p.M : kConfigs[cfg].bm) - 1;
+        const int64_t rb = (p.N < kConfigs[cfg].bn ? p.N : kConfigs[cfg].bn) - 1;
+        if (p.lda > kReach || p.ldb > kReach || (ra * p.lda + p.K) * 2 > kReach ||
+            (rb * p.ldb + p.K) * (p.Bs ? 1 : 2) > kReach)
+            return false;
+    }
+    return true;
+}
+
 // Estimated time: ceil(tiles / concurrent workgroups) waves, each lasting the
 // tile area x workgroups per CU / the per-CU rate, between the 256 x 256
 // tiles (the scheduled K = 64 kernel, config 5: on gfx950 at M = 4608 it runs
@@ -1120,9 +1137,10 @@ int64_t tiles_of(const Problem& p, int cfg) {
 // 128 x 128 tiles.
 // Whole-wave cost model: waves of tiles x tile area x workgroups per CU / rate.
 int pick_by_waves(const Problem* ps, int n, int cus, std::initializer_list<int> cands) {
-    int best = *cands.begin();
+    int best = 1;
     double best_t = 1e300;
     for (int cfg : cands) {
+        if (!reaches(ps, n, cfg)) continue;
         const Config c = kConfigs[cfg];
         int64_t tiles = 0;
         for (int i = 0; i < n; ++i) tiles += tiles_of(ps[i], cfg);
@@ -1412,7 +1430,7 @@ extern "C" int dt_gemm_bf16_ws(const dt_gemm_problem* problem, int32_t c_type, v
     DT_REQUIRE(is_io_type(c_type), "dt_gemm_bf16_ws: c_type %d unsupported", c_type);
     const int rc = validate(q, c_type, &p, &tiled);
     if (rc) return rc;
-    if (!tiled) return dt_gemm_bf16_grouped(problem, 1, c_type, -1, stream);
+    if (!tiled || !reaches(&p, 1, kSplitConfig)) return dt_gemm_bf16_grouped(problem, 1, c_type, -1, stream);
     const int S = split_count(q.M, q.N, q.K, cu_count());
     const int64_t ldp = gemm_split_ld(q.N), blocks = q.K / 64;
     Problem ps[kMaxGroup];

@@ -330,6 +330,39 @@ def test_prepared_launch_keeps_its_scratch(orc, dev):
         assert all((t == 255).all() for t in others), fn.__name__
 
 
+@pytest.mark.parametrize("weights", ["bf16", "q8_0"])
+@pytest.mark.parametrize("M,N,K,lda,ldb", [(128, 3072, 3072, 9_000_000, None), (128, 128, 8192, None, 17_000_000),
+                                           (300, 257, 4160, 9_000_000, None), (256, 65536, 64, 4_300_000, None)])
+def test_gemm_long_rows(dev, M, N, K, lda, ldb, weights):
+    """Rows so far apart that a tile spans more than 2^31 bytes, alone (K ranges)
+    and grouped, against the same operands packed: the sums differ by their order only."""
+    print(f"gemm long rows {weights} {M}x{N}x{K} lda={lda} ldb={ldb}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(SEED + 277)
+    a = torch.randn((M, K), generator=g, device="cuda").bfloat16()
+    w = torch.randn((N, K), generator=g, device="cuda") * 0.02
+
+    def far(t, ld):
+        if ld is None:
+            return t
+        v = torch.empty(t.shape[0] * ld, dtype=t.dtype, device="cuda").as_strided(t.shape, (ld, 1))
+        return v.copy_(t)
+
+    if weights == "q8_0":
+        near = dit_hip.q8_0_split(dit_hip.quantize_q8_0(w).view(-1), N, K)
+        b, one = dit_hip.Q8Weight(far(near.codes, ldb), near.scales), dit_hip.gemm_q8_0
+    else:
+        near, one = w.bfloat16(), dit_hip.gemm
+        b = far(near, ldb and ldb // 2)
+    x = far(a, lda)
+    want = one(a, near, out_dtype=torch.float32)
+    outs = [one(x, b, out_dtype=torch.float32), torch.empty_like(want)]
+    dit_hip.gemm_grouped([(x, b, outs[1])])
+    torch.cuda.synchronize()
+    bound = 1e-5 * want.abs().clamp(min=1.0)  # the file's bar for fp32 output
+    for got in outs:
+        assert ((got - want).abs() <= bound).all(), (got - want).abs().max().item()
+
+
 # ---------------------------------------------------------------- attention --
 def _attn_ref(orc, q, k, v, scale=None):
     """q [B, Sq, H, D] -> oracle attention per batch on the bf16-rounded values."""
