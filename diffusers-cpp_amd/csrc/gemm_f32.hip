@@ -518,11 +518,22 @@ int f32_skinny_launch(const F32Problem* ps, int n, hipStream_t st) {
 int64_t f32_tiles(const F32Problem& p) { return (int64_t)((p.M + FT - 1) / FT) * ((p.N + FT - 1) / FT); }
 
 int f32_launch(const F32Problem* ps, int n, hipStream_t st) {
+    // 16-byte row loads or not is the kernel's, so a group that holds both kinds
+    // is two launches: one unaligned problem does not slow the others.
+    F32Problem part[2][kF32MaxGroup];
+    int np[2] = {0, 0};
+    for (int i = 0; i < n; ++i) {
+        const int kind = ps[i].vec != 0;
+        part[kind][np[kind]++] = ps[i];
+    }
+    if (np[0] && np[1]) {
+        const int rc = f32_launch(part[0], np[0], st);
+        return rc ? rc : f32_launch(part[1], np[1], st);
+    }
+    const bool vec = np[1] > 0;
     int m_max = 0;
     int64_t cols = 0;
-    bool vec = true;
     for (int i = 0; i < n; ++i) {
-        vec = vec && ps[i].vec;
         m_max = m_max > ps[i].M ? m_max : ps[i].M;
         cols += ps[i].N;
     }

@@ -392,6 +392,26 @@ def test_gemm_f32(orc, dev, M, N, K):
     assert_fp32(host(y), orc.linear(a, b, bias) + add, what=f"gemm_f32 {M}x{N}x{K}")
 
 
+def test_gemm_f32_grouped_unaligned(orc, dev):
+    """A group with one member that takes element-wise loads (K = 37, rows off 16
+    bytes): every member is the product it is by itself, bit for bit, the few-row
+    kernel's among them."""
+    probs, outs, alone, keep = [], [], [], []
+    for i, (N, K, off) in enumerate([(96, 256, 0), (64, 37, 0), (130, 512, 0), (40, 128, 1)]):
+        a = dev_tensor(orc.randn(SEED + 400 + i, (5, K + 4)), torch.float32)[:, off:off + K]
+        b = dev_tensor(orc.randn(SEED + 410 + i, (N, K), std=0.02), torch.float32)
+        outs.append(torch.empty((5, N), device="cuda"))
+        alone.append(dit_hip.gemm_f32(a, b))
+        keep += [a, b]
+        probs.append(dit_hip.GemmProblem(a.data_ptr(), a.stride(0), b.data_ptr(), K, outs[-1].data_ptr(), N, None, 0, None,
+                                         5, N, K, None, 0))
+    arr = (dit_hip.GemmProblem * 4)(*probs)
+    dit_hip.check(dit_hip.load().dt_gemm_f32_grouped(arr, 4, dit_hip.stream()), "dt_gemm_f32_grouped")
+    torch.cuda.synchronize()
+    for i, (got, want) in enumerate(zip(outs, alone)):
+        assert torch.equal(got, want), f"member {i}"
+
+
 def _f32_edges(case, M, N, K):
     """Operands around the range in which the fp32 GEMM takes its products in
     bf16 parts: (a, b), the changed rows or columns inside one 128 x 128 tile."""
