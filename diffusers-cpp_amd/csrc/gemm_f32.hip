@@ -153,7 +153,7 @@ template <bool VEC>
 __device__ __forceinline__ void f32_tile_native(const F32Problem& p, uint8_t* smem, int m0, int n0, int wm, int wn,
                                                 f32x16_t (&tot)[2][2]) {
     constexpr int OP = FT * FKP;
-    float* sm = reinterpret_cast<float*>(smem);  // [A | B][128][FKP]
+    float* sm = reinterpret_cast<float*>(smem);  // [2][A | B][128][FKP]
     const int tid = threadIdx.x, lane = tid & 63;
     const int row = tid >> 1, kh = (tid & 1) * 8;
     const float* arow = p.A + (int64_t)min(m0 + row, p.M - 1) * p.lda + kh;
@@ -166,32 +166,43 @@ __device__ __forceinline__ void f32_tile_native(const F32Problem& p, uint8_t* sm
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[0][j][i][e] = acc[1][j][i][e] = tot[j][i][e] = 0.f;
     const int lrow = lane & 31, lk = (lane >> 5) * 8;
-    const int nk = (p.K + FKC - 1) / FKC;
+    const int nk = (p.K + FKC - 1) / FKC, kn = p.K - kh;
+    float4 a0, a1, b0, b1;
+    auto fetch = [&](int kt) {
+        const int k0 = kt * FKC;
+        a0 = load4<VEC>(arow, k0, kn);
+        a1 = load4<VEC>(arow, k0 + 4, kn);
+        b0 = load4<VEC>(brow, k0, kn);
+        b1 = load4<VEC>(brow, k0 + 4, kn);
+    };
+    fetch(0);
+    __syncthreads();  // every wave's reads of the LDS before this tile are done
     for (int kt = 0; kt < nk; ++kt) {
-        const int k0 = kt * FKC, kn = p.K - kh;
-        const float4 a0 = load4<VEC>(arow, k0, kn), a1 = load4<VEC>(arow, k0 + 4, kn);
-        const float4 b0 = load4<VEC>(brow, k0, kn), b1 = load4<VEC>(brow, k0 + 4, kn);
-        __syncthreads();  // every wave's reads of the previous chunk are done
-        float* a = sm + row * FKP + kh;
+        // Two stages: chunk kt is written beside chunk kt - 1, which is still read.
+        float* const stage = sm + (kt & 1) * 2 * OP;
+        float* a = stage + row * FKP + kh;
         *reinterpret_cast<float4*>(a) = a0;
         *reinterpret_cast<float4*>(a + 4) = a1;
         *reinterpret_cast<float4*>(a + OP) = b0;
         *reinterpret_cast<float4*>(a + OP + 4) = b1;
         __syncthreads();
+        if (kt + 1 < nk) fetch(kt + 1);
 #pragma unroll
-        for (int st = 0; st < 8; ++st) {
-            float w[2], x[2];
+        for (int half = 0; half < 2; ++half) {
+            float4 w[2], x[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                w[j] = sm[OP + (wn + 32 * j + lrow) * FKP + lk + st];
-                x[j] = sm[(wm + 32 * j + lrow) * FKP + lk + st];
+                w[j] = *reinterpret_cast<const float4*>(stage + OP + (wn + 32 * j + lrow) * FKP + lk + 4 * half);
+                x[j] = *reinterpret_cast<const float4*>(stage + (wm + 32 * j + lrow) * FKP + lk + 4 * half);
             }
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int st = 0; st < 4; ++st)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    acc[st & 1][j][i] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(w[j], x[i], acc[st & 1][j][i], 0, 0, 0);
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        acc[st & 1][j][i] =
+                            __builtin_amdgcn_mfma_f32_32x32x2f32(w[j][st], x[i][st], acc[st & 1][j][i], 0, 0, 0);
         }
         if ((kt + 1) % FLUSH == 0 || kt + 1 == nk) {
 #pragma unroll
@@ -210,7 +221,7 @@ __device__ __forceinline__ void f32_tile_native(const F32Problem& p, uint8_t* sm
 template <bool VEC>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[XSTAGES * XSTAGE];
-    static_assert(2 * FT * FKP * 4 <= XSTAGES * XSTAGE, "the fp32 tile's stage");
+    static_assert(2 * 2 * FT * FKP * 4 <= XSTAGES * XSTAGE, "the fp32 tile's stages");
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tm, tn;
@@ -295,6 +306,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
             for (int i = 0; i < 2; ++i)
                 c[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], xf[i], c[j][i], 0, 0, 0);
     };
+    // Set by a thread that has staged an operand out of range, at the end of an even or
+    // odd run of FLUSH chunks, and read at the end of the next one: the rest of
+    // the split products is then not taken.  A chunk's barrier lies between every write
+    // and the reads before and after it, so all threads read the same.
+    __shared__ int out_of_range[2];
+    if (tid < 2) out_of_range[tid] = 0;
     fetch(0);
     stash(smem);
     fetch(1);
@@ -302,6 +319,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
     fetch(2);
     __syncthreads();
     uint8_t *s0 = smem, *s1 = smem + XSTAGE, *s2 = smem + 2 * XSTAGE;  // chunk kt, kt + 1, kt + 2
+    bool early = false;
     for (int kt = 0; kt < nk;) {
         const int end = min(kt + FLUSH, nk);
         for (; kt < end; ++kt) {
@@ -339,6 +357,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
                     tot[j][i][e] += acc[j][i][e];
                     acc[j][i][e] = 0.f;
                 }
+        const int run = (kt - 1) / FLUSH & 1;
+        if (!(big < kSplitMax)) out_of_range[run] = 1;
+        if (out_of_range[run ^ 1]) {
+            early = true;
+            break;
+        }
     }
 
     // The split products stand in for fp32 ones only where every part of
@@ -347,6 +371,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
     // sum of operands that are all zero or at least 2^-35 is exact however
     // small, so a small sum first looks for smaller operands.
     bool odd = !(big < kSplitMax), small = false;
+    // One or two products (element-wise loads): leaving out the smallest three of nine then
+    // shows, up to 1.9 of fp32's half units instead of 1.
+    if constexpr (!VEC) odd |= K < 3;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -357,7 +384,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const F32Group grp) {
                 odd |= !(fabsf(v) < INFINITY);
                 small |= fabsf(v) < kSplitMin;
             }
-    if (__syncthreads_or(small)) {
+    if (!early && __syncthreads_or(small)) {
         for (int kt = 0; kt < nk; ++kt) {
             fetch(kt);
 #pragma unroll

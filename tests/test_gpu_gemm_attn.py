@@ -461,6 +461,37 @@ def test_gemm_f32_operand_range(dev, case, M, N, K):
         assert (np.abs(got[ok] - ref[ok]) <= bound).all(), np.max(np.abs(got[ok] - ref[ok]) / bound)
 
 
+@pytest.mark.parametrize("K", [1, 2, 3])
+def test_gemm_f32_few_terms(dev, K):
+    """One, two and three products, whose roundings nothing hides: within K
+    fp32 roundings of the sum of magnitudes (K = 1: the rounded product)."""
+    print(f"gemm_f32 K={K}", flush=True)
+    rng = np.random.default_rng(SEED + 285)
+    a, b = ((1.0 + 0.02 * rng.random((300, K))).astype(np.float32) for _ in "ab")
+    got = host(dit_hip.gemm_f32(dev_tensor(a, torch.float32), dev_tensor(b, torch.float32))).astype(np.float64)
+    ref = a.astype(np.float64) @ b.astype(np.float64).T
+    if K == 1:
+        assert np.array_equal(got, ref.astype(np.float32).astype(np.float64))
+    assert (np.abs(got - ref) <= K * 2.0 ** -24 * np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T).all()
+
+
+@pytest.mark.parametrize("k", [0, 127, 128, 300, 1039])
+def test_gemm_f32_large_operand_at(dev, k):
+    """One operand out of the split's range at k: its tile leaves the split products at
+    the end of a run of 128 k, or after the last; the other tiles keep them."""
+    print(f"gemm_f32 large operand at k={k}", flush=True)
+    rng = np.random.default_rng(SEED + 286)
+    M, N, K = 200, 150, 1040
+    a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    plain = host(dit_hip.gemm_f32(dev_tensor(a, torch.float32), dev_tensor(b, torch.float32)))
+    a[3, k] *= np.float32(2.0 ** 45)
+    got = host(dit_hip.gemm_f32(dev_tensor(a, torch.float32), dev_tensor(b, torch.float32)))
+    assert np.array_equal(got[128:], plain[128:])
+    ref = a.astype(np.float64) @ b.astype(np.float64).T
+    mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+    assert (np.abs(got - ref) <= K * 2.0 ** -24 * mag).all()
+
+
 def test_gemm_f32_strided_in_place(orc, dev):
     """lda = K + 4, C written into a wider buffer, and C aliasing the addend."""
     M, N, K = 200, 96, 256
