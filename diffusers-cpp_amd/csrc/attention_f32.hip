@@ -70,14 +70,14 @@ struct F32Attn {
     const float* v;
     float* o;
     int64_t qs[3], ks[3], vs[3], os[3];  // batch, token, head strides (elements)
-    int32_t bh, heads, seq_q, seq_kv, q_blocks, kv_blocks;
+    int32_t bh, bh0, heads, seq_q, seq_kv, q_blocks, kv_blocks;  // bh (batch, head) pairs from bh0 on
     float scale, c_hi, c_lo;             // scale * log2(e) = c_hi + c_lo
-    uint8_t* kp;                         // planes [batch * heads][seq_kv][3][128] bf16
+    uint8_t* kp;                         // planes [bh][seq_kv][3][128] bf16
     uint8_t* vp;
-    uint32_t* flags;                     // [batch * heads][2 kv_blocks]: 1 = operands out of range
+    uint32_t* flags;                     // [bh][2 kv_blocks]: 1 = operands out of range
     int32_t splits;                      // key ranges per query block; > 1: partial results
-    float* part;                         // [split][batch * heads][seq_q][128]: O before its division by l
-    float2* ml;                          // [split][batch * heads][seq_q]: (m, l)
+    float* part;                         // [split][bh][seq_q][128]: O before its division by l
+    float2* ml;                          // [split][bh][seq_q]: (m, l)
 };
 
 // 8 fp32 as three planes of 8 bf16.
@@ -105,7 +105,7 @@ __device__ __forceinline__ void load8(const float* p, float (&x)[8]) {
 // Block (i, bh, z): rows [64 i, + 64) of K (z = 0) or V (z = 1) of one head, and whether
 // any of them is out of range.
 __global__ __launch_bounds__(256) void split_kv_kernel(const F32Attn a) {
-    const int bh = blockIdx.y, h = bh % a.heads, b = bh / a.heads;
+    const int bh = blockIdx.y, h = (a.bh0 + bh) % a.heads, b = (a.bh0 + bh) / a.heads;
     const bool is_v = blockIdx.z != 0;
     const float* src = is_v ? a.v + b * a.vs[0] + h * a.vs[2] : a.k + b * a.ks[0] + h * a.ks[2];
     const int64_t ts = is_v ? a.vs[1] : a.ks[1];
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_f32_kernel(const F32Attn a)
     if ((nb & 7u) == 0) bid = (bid & 7u) * (nb >> 3) + (bid >> 3);  // a run of heads per XCD
     const int qblk = (int)(bid % (uint32_t)a.q_blocks);
     const int split = (int)(bid / (uint32_t)a.q_blocks) % a.splits, bh = (int)(bid / (uint32_t)(a.q_blocks * a.splits));
-    const int h = bh % a.heads, b = bh / a.heads;
+    const int h = (a.bh0 + bh) % a.heads, b = (a.bh0 + bh) / a.heads;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
     const int q = qblk * QB + wave * 32 + r;
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const F32Attn a) {
         o.z += w * p.z;
         o.w += w * p.w;
     }
-    const int64_t bh = row / a.seq_q, q = row - bh * a.seq_q, b = bh / a.heads, h = bh - b * a.heads;
+    const int64_t bh = row / a.seq_q, q = row - bh * a.seq_q, b = (a.bh0 + bh) / a.heads, h = a.bh0 + bh - b * a.heads;
     const float inv = 1.0f / l;
     *reinterpret_cast<float4*>(a.o + b * a.os[0] + q * a.os[1] + h * a.os[2] + d) =
         make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
@@ -538,8 +538,20 @@ int attn_f32_splits(int64_t bh, int64_t seq_q, int64_t seq_kv) {
 
 }  // namespace
 
-size_t attn_f32_fused_bytes(int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_kv) {
-    const int64_t bh = batch * heads, blocks = (seq_kv + SPLIT_ROWS - 1) / SPLIT_ROWS;
+// Largest number of (batch, head) pairs, in launches of about equal size, whose
+// workspace is at most `limit`; 0: not even one's.
+int64_t attn_f32_fused_heads(int64_t bh, int64_t seq_q, int64_t seq_kv, size_t limit) {
+    int64_t n = (int64_t)(limit / (size_t)(2 * seq_kv * ROWB));
+    if (n > bh) n = bh;
+    if (n > 65535) n = 65535;  // split_kv_kernel's grid
+    while (n > 0 && attn_f32_fused_bytes(n, seq_q, seq_kv) > limit) --n;
+    if (n == 0) return 0;
+    const int64_t launches = (bh + n - 1) / n, even = (bh + launches - 1) / launches;
+    return attn_f32_fused_bytes(even, seq_q, seq_kv) <= limit ? even : n;  // fewer heads may take more key ranges
+}
+
+size_t attn_f32_fused_bytes(int64_t bh, int64_t seq_q, int64_t seq_kv) {
+    const int64_t blocks = (seq_kv + SPLIT_ROWS - 1) / SPLIT_ROWS;
     const int64_t splits = attn_f32_splits(bh, seq_q, seq_kv);
     return (size_t)(bh * (2 * seq_kv * ROWB + 8 * blocks)) + (splits > 1 ? (size_t)(splits * bh * seq_q * (D * 4 + 8)) : 0);
 }
@@ -552,12 +564,12 @@ bool attn_f32_fused_takes(const float* q, const float* k, const float* v, const 
         return false;
     for (int i = 0; i < 3; ++i)
         if (qs[i] % 4 || ks[i] % 4 || vs[i] % 4 || os[i] % 4) return false;
-    return batch * heads <= 65535 && ((seq_q + QB - 1) / QB) * batch * heads < (1ll << 31) && seq_kv < (1ll << 30);
+    return batch * heads < (1ll << 31) && ((seq_q + QB - 1) / QB) * batch * heads < (1ll << 31) && seq_kv < (1ll << 30);
 }
 
 int attn_f32_fused(const float* q, const float* k, const float* v, float* o, int64_t batch, int64_t heads,
                    int64_t seq_q, int64_t seq_kv, const int64_t* qs, const int64_t* ks, const int64_t* vs,
-                   const int64_t* os, float scale, void* workspace, hipStream_t st) {
+                   const int64_t* os, float scale, int64_t heads_per_launch, void* workspace, hipStream_t st) {
     F32Attn a{};
     a.q = q;
     a.k = k;
@@ -569,7 +581,6 @@ int attn_f32_fused(const float* q, const float* k, const float* v, float* o, int
         a.vs[i] = vs[i];
         a.os[i] = os[i];
     }
-    a.bh = (int32_t)(batch * heads);
     a.heads = (int32_t)heads;
     a.seq_q = (int32_t)seq_q;
     a.seq_kv = (int32_t)seq_kv;
@@ -580,21 +591,28 @@ int attn_f32_fused(const float* q, const float* k, const float* v, float* o, int
     a.c_hi = (float)c;
     a.c_lo = (float)(c - (double)a.c_hi);
     a.kp = (uint8_t*)workspace;
-    a.vp = a.kp + (size_t)(batch * heads) * (size_t)seq_kv * ROWB;
-    a.splits = attn_f32_splits(batch * heads, seq_q, seq_kv);
-    const size_t rows = a.splits > 1 ? (size_t)a.splits * (size_t)(batch * heads) * (size_t)seq_q : 0;
-    a.part = (float*)(a.vp + (size_t)(batch * heads) * (size_t)seq_kv * ROWB);
-    a.ml = (float2*)(a.part + rows * D);
-    a.flags = (uint32_t*)(a.ml + rows);
-    hipLaunchKernelGGL(split_kv_kernel, dim3((unsigned)a.kv_blocks, (unsigned)(batch * heads), 2), dim3(256), 0, st, a);
-    const int rc = check_launch("dt_flash_attn_f32(split)");
-    if (rc) return rc;
-    hipLaunchKernelGGL(flash_attn_f32_kernel, dim3((unsigned)(a.q_blocks * batch * heads * a.splits)), dim3(256), 0, st,
-                       a);
-    const int rk = check_launch("dt_flash_attn_f32");
-    if (rk || a.splits == 1) return rk;
-    hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)((batch * heads * seq_q + 7) / 8)), dim3(256), 0, st, a);
-    return check_launch("dt_flash_attn_f32(combine)");
+    for (int64_t bh0 = 0; bh0 < batch * heads; bh0 += heads_per_launch) {
+        const int64_t bh = batch * heads - bh0 < heads_per_launch ? batch * heads - bh0 : heads_per_launch;
+        a.bh0 = (int32_t)bh0;
+        a.bh = (int32_t)bh;
+        a.vp = a.kp + (size_t)bh * (size_t)seq_kv * ROWB;
+        a.splits = attn_f32_splits(heads_per_launch, seq_q, seq_kv);  // what the workspace is sized for
+        const size_t rows = a.splits > 1 ? (size_t)a.splits * (size_t)bh * (size_t)seq_q : 0;
+        a.part = (float*)(a.vp + (size_t)bh * (size_t)seq_kv * ROWB);
+        a.ml = (float2*)(a.part + rows * D);
+        a.flags = (uint32_t*)(a.ml + rows);
+        hipLaunchKernelGGL(split_kv_kernel, dim3((unsigned)a.kv_blocks, (unsigned)bh, 2), dim3(256), 0, st, a);
+        int rc = check_launch("dt_flash_attn_f32(split)");
+        if (rc) return rc;
+        hipLaunchKernelGGL(flash_attn_f32_kernel, dim3((unsigned)(a.q_blocks * bh * a.splits)), dim3(256), 0, st, a);
+        rc = check_launch("dt_flash_attn_f32");
+        if (rc) return rc;
+        if (a.splits == 1) continue;
+        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)((bh * seq_q + 7) / 8)), dim3(256), 0, st, a);
+        rc = check_launch("dt_flash_attn_f32(combine)");
+        if (rc) return rc;
+    }
+    return DT_OK;
 }
 
 }  // namespace dit

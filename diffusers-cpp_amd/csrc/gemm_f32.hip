@@ -741,18 +741,33 @@ extern "C" int dt_gemm_f32_ws(const dt_gemm_problem* problem, void* workspace, s
 
 // Workspace of dt_flash_attn_f32: per head of a group of up to 8, the
 // scores [seq_q][seq_kv] and V^T [head_dim][seq_kv], fp32; or what the fused kernel
-// needs, if that is more.
+// needs, if that is more.  It takes 1536 bytes per key and head, so beyond
+// kFusedWs (24 heads of 7000 keys) and the group's scores it takes fewer heads
+// per launch: a call's memory does not grow with its batch.
 static int64_t attn_f32_group(int64_t batch, int64_t heads) {
     const int64_t bh = batch * heads;
     return bh < dit::kF32MaxGroup ? bh : dit::kF32MaxGroup;
+}
+constexpr size_t kFusedWs = 256u << 20;
+
+static size_t attn_f32_gemm_bytes(int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_kv, int64_t head_dim) {
+    const int64_t per = (seq_q * seq_kv + head_dim * seq_kv + 3) / 4 * 4;  // 16-byte aligned per head
+    return (size_t)(attn_f32_group(batch, heads) * per) * sizeof(float);
+}
+
+// (batch, head) pairs per launch of the fused kernel, 0: not for these sizes.
+static int64_t attn_f32_per_launch(int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_kv, int64_t head_dim) {
+    if (head_dim != 128) return 0;
+    const size_t gemms = attn_f32_gemm_bytes(batch, heads, seq_q, seq_kv, head_dim);
+    return dit::attn_f32_fused_heads(batch * heads, seq_q, seq_kv, gemms > kFusedWs ? gemms : kFusedWs);
 }
 
 extern "C" size_t dt_flash_attn_f32_workspace_bytes(int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_kv,
                                                      int64_t head_dim) {
     if (batch <= 0 || heads <= 0 || seq_q <= 0 || seq_kv <= 0 || head_dim <= 0) return 0;
-    const int64_t per = (seq_q * seq_kv + head_dim * seq_kv + 3) / 4 * 4;  // 16-byte aligned per head
-    const size_t gemms = (size_t)(attn_f32_group(batch, heads) * per) * sizeof(float);
-    const size_t fused = head_dim == 128 ? dit::attn_f32_fused_bytes(batch, heads, seq_q, seq_kv) : 0;
+    const size_t gemms = attn_f32_gemm_bytes(batch, heads, seq_q, seq_kv, head_dim);
+    const int64_t n = attn_f32_per_launch(batch, heads, seq_q, seq_kv, head_dim);
+    const size_t fused = n ? dit::attn_f32_fused_bytes(n, seq_q, seq_kv) : 0;
     return gemms > fused ? gemms : fused;
 }
 
@@ -773,10 +788,11 @@ extern "C" int dt_flash_attn_f32(const float* q, const float* k, const float* v,
     DT_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
                "dt_flash_attn_f32: workspace of %zu bytes (16-byte aligned) needed", need);
     hipStream_t st = (hipStream_t)stream;
-    if (attn_f32_fused_takes(q, k, v, o, batch, heads, seq_q, seq_kv, head_dim, q_strides, k_strides, v_strides, o_strides,
-                             scale))
+    const int64_t per_launch = attn_f32_per_launch(batch, heads, seq_q, seq_kv, head_dim);
+    if (per_launch && attn_f32_fused_takes(q, k, v, o, batch, heads, seq_q, seq_kv, head_dim, q_strides, k_strides,
+                                           v_strides, o_strides, scale))
         return attn_f32_fused(q, k, v, o, batch, heads, seq_q, seq_kv, q_strides, k_strides, v_strides, o_strides, scale,
-                              workspace, st);
+                              per_launch, workspace, st);
     const int64_t per = (seq_q * seq_kv + head_dim * seq_kv + 3) / 4 * 4;
     const int64_t bh = batch * heads, gsz = attn_f32_group(batch, heads);
     float* ws = (float*)workspace;

@@ -89,14 +89,16 @@ int gemm_reduce(const float* part, int S, int64_t M, int64_t N, void* C, int64_t
                 const void* addend, int64_t ldd, int32_t c_type, hipStream_t st);
 
 // Fused fp32 attention (attention_f32.hip) for head_dim 128 with 16-byte rows:
-// whether it takes a call, its workspace, the launches.
+// whether it takes a call, the (batch, head) pairs it takes per launch within a
+// workspace limit, their workspace, the launches.
 bool attn_f32_fused_takes(const float* q, const float* k, const float* v, const float* o, int64_t batch, int64_t heads,
                           int64_t seq_q, int64_t seq_kv, int64_t head_dim, const int64_t* qs, const int64_t* ks,
                           const int64_t* vs, const int64_t* os, float scale);
-size_t attn_f32_fused_bytes(int64_t batch, int64_t heads, int64_t seq_q, int64_t seq_kv);
+int64_t attn_f32_fused_heads(int64_t bh, int64_t seq_q, int64_t seq_kv, size_t limit);
+size_t attn_f32_fused_bytes(int64_t bh, int64_t seq_q, int64_t seq_kv);
 int attn_f32_fused(const float* q, const float* k, const float* v, float* o, int64_t batch, int64_t heads,
                    int64_t seq_q, int64_t seq_kv, const int64_t* qs, const int64_t* ks, const int64_t* vs,
-                   const int64_t* os, float scale, void* workspace, hipStream_t st);
+                   const int64_t* os, float scale, int64_t heads_per_launch, void* workspace, hipStream_t st);
 
 // Backend accessors (capi.cpp).
 hipStream_t backend_stream(dt_backend* be);

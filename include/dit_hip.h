@@ -430,7 +430,8 @@ int dt_flash_attn_qk_bf16(const void *q0, const int64_t *q0_strides, const float
  * dt_flash_attn_f32: softmax(scale Q K^T) V per (batch, head), strides as
  * dt_flash_attn_bf16, fp32 o; K's and V's parts (head_dim 128, 16-byte aligned
  * rows) or the scores of up to 8 heads at a time go through `workspace`
- * (dt_flash_attn_f32_workspace_bytes, 16-byte aligned). */
+ * (dt_flash_attn_f32_workspace_bytes, 16-byte aligned), in groups of heads, so it
+ * needs at most 256 MB or what the scores of 8 heads take. */
 int dt_gemm_f32(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int64_t M,
                 int64_t N, int64_t K, const float *bias, const float *addend, int64_t ldd, dt_stream_t stream);
 int dt_gemm_f32_grouped(const dt_gemm_problem *problems, int32_t count, dt_stream_t stream);

@@ -122,6 +122,16 @@ def test_rope_table_matches_oracle_cache(orc):
         assert np.array_equal(tab2[p], orc.rope_cache(float(p), 2, 2, 2000.0))
 
 
+def test_flash_attn_f32_workspace_bytes():
+    """Bounded by eight heads' scores and V^T or 256 MB, whatever the number of heads;
+    a small call's parts of K and V (1536 bytes per key and head) fit whole."""
+    lib = dit_hip.load()
+    for B, H, Sq, Skv in [(1, 64, 32, 65536), (16, 24, 4608, 4608), (1, 1, 1, 1 << 20), (4096, 24, 1, 300), (1, 3, 5, 200000)]:
+        scores = min(B * H, 8) * ((Sq + 128) * Skv + 3) // 4 * 4 * 4
+        assert lib.dt_flash_attn_f32_workspace_bytes(B, H, Sq, Skv, 128) <= max(scores, 256 << 20), (B, H, Sq, Skv)
+    assert lib.dt_flash_attn_f32_workspace_bytes(1, 24, 320, 320, 128) >= 24 * 1536 * 320
+
+
 def test_groupnorm_workspace_bytes():
     lib = dit_hip.load()
     # one (K, sum, sumsq per chunk) record per (n, g), chunks of 1024 elements (the scalar path's)

@@ -655,6 +655,25 @@ def test_flash_attn_f32_large_scale(dev, up):
     assert ((got - ref).abs() <= min(bound, 0.25) * vd.abs().max()).all(), (got - ref).abs().max().item()
 
 
+@pytest.mark.parametrize("B,Sq,Skv,H", [(1, 3, 4100, 47), (2, 130, 7000, 13)])
+def test_flash_attn_f32_workspace_groups(dev, B, Sq, Skv, H):
+    """Heads whose K and V parts pass the workspace's bound are taken in several
+    launches (an odd count: the last one smaller): the bound holds, and each
+    (batch, head) is its attention in 64 bits."""
+    print(f"attn_f32 groups B={B} Sq={Sq} Skv={Skv} H={H}", flush=True)
+    parts, scores = B * H * 1536 * Skv, 8 * 4 * (Sq + 128) * Skv
+    assert parts > max(scores, 256 << 20) >= dit_hip.load().dt_flash_attn_f32_workspace_bytes(B, H, Sq, Skv, 128)
+    g = torch.Generator(device="cuda").manual_seed(SEED + 296)
+    q, k, v = (torch.randn((B, S, H, 128), generator=g, device="cuda") for S in (Sq, Skv, Skv))
+    o = dit_hip.flash_attn_f32(q, k, v)
+    torch.cuda.synchronize()
+    for b in range(B):
+        for h in range(H):
+            p = torch.softmax(q[b, :, h].double() @ k[b, :, h].double().t().contiguous() / 128 ** 0.5, -1)
+            ref = p @ v[b, :, h].double()
+            assert ((o[b, :, h].double() - ref).abs() <= 1e-5).all(), (b, h)
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,Sq,Skv,H", ATTN_SHAPES)
 def test_flash_attn(orc, dev, B, Sq, Skv, H, out_dtype):
