@@ -1041,7 +1041,8 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
                      aligned16(ws) && (!stats || (a.cg >= 4 && a.cg <= 64));
     int64_t tiles_w, tiles_h;
     DT_REQUIRE(!gn || dma, "%s: the GroupNorm fold needs a 3x3 conv with a workspace", what);
-    if (dma && !stats && conv_is_direct(K, io_type, upscale2, x, N, Ci, H * W, y, Co)) {
+    // The GroupNorm fold is the copy's to apply.
+    if (dma && !stats && !gn && conv_is_direct(K, io_type, upscale2, x, N, Ci, H * W, y, Co)) {
         // One row of H W pixels (a 1x1 conv has no rows of its own).
         a.TR = 1;
         a.TC = kPwPx;

@@ -6,6 +6,8 @@ reference is the oracle on the bf16-rounded input and weights: fp32 outputs
 are held to |d| <= 1e-5 * max(|ref|, 1) (only the fp32 accumulation order
 differs), bf16 outputs to the bf16 bar (rel L2 <= 1e-2, cos >= 0.9999) plus
 one bf16 ulp for the single output rounding."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -401,6 +403,39 @@ def test_conv2d_tiles_and_residual(orc, dev, shape, co, k, io):
     check(host(y), ref, io, f"conv2d {shape} -> {co}")
     check(host(staged), ref, io, f"conv2d staged {shape} -> {co}")
     check(host(out), (as_input(res, io) + ref) * np.float32(0.5), io, "conv + residual", one_rounding=False)
+
+
+def test_conv2d_1x1_groupnorm_fold(orc, dev):
+    """conv2d_fold with a GroupNorm + SiLU on a 1x1 whose plane the kernel without
+    the channel-last copy would take: the copy applies it, as GroupNorm and conv apart."""
+    lib = dit_hip.load()
+    N, ci, H, W, co, G = 1, 64, 32, 40, 96, 32
+    x = dev_tensor(orc.randn(SEED + 99, (N, ci, H, W), mean=0.3), torch.bfloat16)
+    gw, gb = (dev_tensor(orc.randn(SEED + 100 + i, (ci,), mean=1.0 - i, std=0.1), torch.float32) for i in range(2))
+    wp = dit_hip.conv2d_pack(dev_tensor(orc.randn(SEED + 102, (co, ci, 1, 1), std=0.1), torch.float32))
+    want = dit_hip.conv2d(dit_hip.groupnorm_silu(x, G, gw, gb, 1e-6), wp)
+
+    class Fold(ctypes.Structure):  # dit::ConvFold (kernels.hpp)
+        _fields_ = [("mr", ctypes.c_void_p), ("w", ctypes.c_void_p), ("b", ctypes.c_void_p), ("groups", ctypes.c_int),
+                    ("silu", ctypes.c_int), ("res", ctypes.c_void_p), ("mode", ctypes.c_int), ("scale", ctypes.c_float)]
+
+    c64, ptr, i32 = ctypes.c_int64, ctypes.c_void_p, ctypes.c_int32
+    mean_rstd = getattr(lib, "_ZN3dit12gn_mean_rstdEPKvllllfPvP15HIP_vector_typeIfLj2EEiP12ihipStream_t")
+    fold_call = getattr(lib, "_ZN3dit11conv2d_foldEPKvllllS1_lliPKfRKNS_8ConvFoldEPvS7_miP12ihipStream_t")
+    mean_rstd.argtypes = [ptr, c64, c64, c64, c64, ctypes.c_float, ptr, ptr, i32, ptr]
+    fold_call.argtypes = [ptr, c64, c64, c64, c64, ptr, c64, c64, i32, ptr, ctypes.POINTER(Fold), ptr, ptr,
+                          ctypes.c_size_t, i32, ptr]
+    mr = torch.empty((N * G, 2), device="cuda")
+    gws = torch.empty(lib.dt_groupnorm_workspace_bytes(N, ci, H * W, G), dtype=torch.uint8, device="cuda")
+    ws = torch.empty(lib.dt_conv2d_workspace_bytes(N, ci, H, W), dtype=torch.uint8, device="cuda")
+    y = torch.empty((N, co, H, W), dtype=torch.bfloat16, device="cuda")
+    st = dit_hip.stream()
+    dit_hip.check(mean_rstd(x.data_ptr(), N, ci, H * W, G, 1e-6, gws.data_ptr(), mr.data_ptr(), dit_hip.BF16, st))
+    f = Fold(mr.data_ptr(), gw.data_ptr(), gb.data_ptr(), G, 1, None, 0, 1.0)
+    dit_hip.check(fold_call(x.data_ptr(), N, ci, H, W, wp.packed.data_ptr(), co, 1, 0, None, ctypes.byref(f), y.data_ptr(),
+                            ws.data_ptr(), ws.numel(), dit_hip.BF16, st))
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
 
 
 def test_conv2d_1x1_in_place(orc, dev):
