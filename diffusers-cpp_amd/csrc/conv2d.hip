@@ -978,14 +978,13 @@ void conv_geometry(int64_t Hs, int64_t Ws, int* TR, int* TC, int64_t* tiles_w, i
 
 int64_t nhwc_elems(int64_t N, int64_t Ci, int64_t H, int64_t W) { return N * H * W * pad_to(Ci, kCi2); }
 
-// Tile geometry of the DMA kernel: 256-pixel tiles, TC = 256 .. 16 columns.
-// The DMA kernel's 256-pixel tile: 8 rows of 32 (16 x 16 on narrower
-// images).  Its input patch is then 10 x 34 records against 3 x 258 for a
+// Tile geometry of the DMA kernel: tiles of px pixels (128, 256 or 512; conv_launch
+// says which), rows of 32 (of 16 on narrower images): 4 x 32, 8 x 32 or 16 x 32.  The
+// 8 x 32 tile's input patch is then 10 x 34 records against 3 x 258 for a
 // 1 x 256 strip, and on gfx950 it ran 3-22% faster than the 1 x 256, 2 x 128
 // and 4 x 64 tiles at every decoder shape ([1,128,1024,1024] -> 128 bf16:
 // 784 / 760 / 765 us against 701 us, channel-last copy included), with the
 // same output bits.
-// px: the tile's pixels, 256 or 512 (16 x 32).
 void conv_geometry2(int64_t Hs, int64_t Ws, int px, int* TR, int* TC, int64_t* tiles_w, int64_t* tiles_h) {
     *TC = Ws >= 32 ? 32 : 16;
     *TR = px / *TC;
@@ -1054,11 +1053,15 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
         else hipLaunchKernelGGL(conv1x1_kernel<false>, g1, dim3(512), 0, st, a, H * W);
         return check_launch(what);
     }
-    // The largest pixel tile that still gives every CU a workgroup (half the
-    // weight DMA per output pixel for each doubling), by tiles of the whole launch:
-    // 512 pixels from one per CU ([1,256,256,256] -> 256, 256 tiles: 95 us against 106
-    // at 256 pixels), 256 from more than one per two CUs, else 128
-    // ([1,512,64,64] -> 512, 64 tiles of 256: 55 us against 73; [1,512,32,32]: 51 and 68).
+    // Pixel tile: 512, 256 or 128, by rounds of one workgroup per CU.  A tile of half the
+    // pixels has the same weights to load, so its round takes 0.57 of a 512-pixel one's and
+    // 0.42 at 128 pixels ([1,256,256,256] -> 256, 256 tiles of 512: 92 us, 512 of 256: 2 x 51;
+    // [1,512,64,64] -> 512, 64 of 256: 72, 128 of 128: 53); the last, partial round decides
+    // ([1,256,300,470] -> 128: 285 tiles of 512 take 215 us, 570 of 256 194; [1,512,160,160] ->
+    // 512: 200 of 512 143, 400 of 256 164; [1,512,96,96]: 144 of 256 76, 288 of 128 101).
+    // A 1x1 has a ninth of the work per tile and several workgroups per CU, and memory bounds
+    // it: 512 pixels from one tile per CU ([1,128,301,301] -> 128, 190 of them: 61 us, 361 of
+    // 256: 56), 256 from more than one per two CUs.
     int px = 256;
     if (dma && !stats) {
         auto tiles = [&](int p) {
@@ -1067,8 +1070,11 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
             conv_geometry2(Hs, Ws, p, &tr, &tc, &tw, &th);
             return tw * th * ((Co + kTileCo - 1) / kTileCo) * N;
         };
-        const int cus = cu_count();
-        px = tiles(512) >= cus ? 512 : tiles(256) > cus / 2 ? 256 : 128;
+        const int64_t cus = cu_count();
+        auto rounds = [&](int p) { return (double)((tiles(p) + cus - 1) / cus); };
+        if (K == 1) px = tiles(512) >= cus ? 512 : tiles(256) > cus / 2 ? 256 : 128;
+        else if (rounds(512) <= 0.57 * rounds(256)) px = 512;
+        else px = rounds(256) <= 0.74 * rounds(128) ? 256 : 128;  // 0.42 / 0.57
     }
     if (dma) conv_geometry2(Hs, Ws, px, &a.TR, &a.TC, &tiles_w, &tiles_h);
     else conv_geometry(Hs, Ws, &a.TR, &a.TC, &tiles_w, &tiles_h);

@@ -356,13 +356,13 @@ def test_groupnorm_folded_into_conv_equals_the_nodes(orc, dev, io, shape, G, co,
     check(host(fused_out), want, io, "GroupNorm + conv", one_rounding=False)
 
 
-# 512-pixel tiles (16 x 32) are taken when they still give every CU a workgroup
-# (N x tiles x output-channel tiles >= 256); these shapes reach them,
-# with a batch, a partial output-channel tile, a partial column tile and the
-# 2x upscale.
+# 512-pixel tiles (16 x 32) are taken where the rounds of one workgroup per CU they
+# make are few enough; these shapes reach them on 256 CUs (512 tiles, and 425 with a
+# partial column tile; 544 make a third round and take 256 pixels), with a batch, a
+# partial output-channel tile and the 2x upscale.
 @pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape,co,up2", [((4, 16, 256, 256), 24, False), ((1, 8, 512, 520), 16, False),
-                                          ((1, 16, 256, 256), 8, True)])
+                                          ((1, 16, 256, 256), 8, True), ((1, 8, 400, 520), 16, False)])
 def test_conv2d_512_pixel_tiles(orc, dev, shape, co, up2, io):
     print(f"conv2d 512px x={shape} co={co} up2={up2} {io}", flush=True)
     x = orc.randn(SEED + 90, shape)
@@ -376,10 +376,11 @@ def test_conv2d_512_pixel_tiles(orc, dev, shape, co, up2, io):
 
 
 # The pixel tiles of the launch rule and the direct 1x1, at ragged edges, plain
-# and with the residual epilogue: the values a 256-CU card picks 512, 256 and
-# 128 pixels at, and 1x1 planes that end inside a 256-pixel tile.
+# and with the residual epilogue: the values a 256-CU card picks 256 (306 tiles of 512
+# are two rounds, 612 of 256 three), 512, 256 and 128 pixels at, and 1x1 planes that
+# end inside a 256-pixel tile.
 @pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("shape,co,k", [((1, 32, 270, 266), 200, 3), ((1, 32, 150, 133), 130, 3),
+@pytest.mark.parametrize("shape,co,k", [((1, 32, 270, 266), 200, 3), ((1, 32, 200, 266), 200, 3), ((1, 32, 150, 133), 130, 3),
                                         ((1, 48, 37, 30), 140, 3), ((2, 32, 36, 30), 130, 1), ((1, 96, 29, 40), 128, 1),
                                         ((1, 32, 1, 1032), 4, 1)])
 def test_conv2d_tiles_and_residual(orc, dev, shape, co, k, io):
