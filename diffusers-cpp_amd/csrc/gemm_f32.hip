@@ -9,8 +9,11 @@
 // do not: each operand is split exactly into three bf16 parts, x = x0 + x1 +
 // x2 (8 + 8 + 8 bits, each the rounded remainder of the last), and the product
 // taken as the six bf16 MFMAs x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0 with
-// fp32 accumulation.  The three left out are below 2^-26 of |x w|, under fp32's
-// own rounding of one product.  x0 w0 is summed by itself, in runs of 128 k
+// fp32 accumulation.  The three left out are 2^-27.4 of |x w| in the root mean square
+// (N(0, 1) operands) and at most 2^-24.05, about what fp32 rounds one product by, so a
+// product that stands alone may be off by 1.85 half units instead of 1 (K = 1 and 2
+// therefore run on the fp32 matrix cores); from three terms on the total, whose
+// sums are rounded less often, is closer than the fp32 MFMAs' in both measures.  x0 w0 is summed by itself, in runs of 128 k
 // that are then added to the tile's total, and the five small ones in an
 // accumulator of their own, whose rounding is 2^-8 of the other's; so the sum
 // is rounded about 8 + K/128 times where the fp32 MFMA's was 64 + K/128.
