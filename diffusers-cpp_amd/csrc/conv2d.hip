@@ -1124,15 +1124,10 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
         else DT_CONV2_ONE(TT, KS, false, RS, 1, 8);              \
     } while (0)
         if (io_type == DT_TYPE_F32) {
-            if (K == 1) {
-                if (stats) DT_CONV2_LAUNCH(float, 1, true, false);
-                else if (res_mode) DT_CONV2_LAUNCH(float, 1, false, true);
-                else DT_CONV2_LAUNCH(float, 1, false, false);
-            } else {
-                if (stats) DT_CONV2_LAUNCH(float, 3, true, false);
-                else if (res_mode) DT_CONV2_LAUNCH(float, 3, false, true);
-                else DT_CONV2_LAUNCH(float, 3, false, false);
-            }
+            // 3x3 only (conv_uses_dma)
+            if (stats) DT_CONV2_LAUNCH(float, 3, true, false);
+            else if (res_mode) DT_CONV2_LAUNCH(float, 3, false, true);
+            else DT_CONV2_LAUNCH(float, 3, false, false);
         } else {
             if (K == 1) {
                 if (stats) DT_CONV2_LAUNCH(bf16, 1, true, false);

@@ -1087,11 +1087,11 @@ struct Config {
 // 5: config 2 with the operand reads interleaved into the MFMA stream; 6: the
 // same at 224 x 256; 7: config 5 with Q8_0 weights dequantised as they are
 // staged; 8, 9: configs 5 and 7 in eight waves of 128 x 64 (two per SIMD).
-// Chosen by size only, not by callers: 10: few rows (gemm_skinny_kernel); 11: 128 x 128
-// in two k-groups (the rate puts it below config 1's pair of tiles per CU only
-// while one round of it holds every tile).
+// Chosen by size only, not by callers: 10: 128 x 128 in two k-groups (the rate puts it
+// below config 1's pair of tiles per CU only while one round of it holds every
+// tile); 11: few rows (gemm_skinny_kernel, which has no tiles and no row here).
 constexpr int kAnyConfig = 4, kLastConfig = 9;
-constexpr int kSkinnyConfig = 10, kSplitConfig = 11;
+constexpr int kSplitConfig = 10, kSkinnyConfig = 11;
 // Rows up to which the weight stream wins (Python call included, bf16 / Q8_0; the
 // tiles, K split where it is): 18432 x 3072 at 16 rows 37.9 / 27.5 us against 40.7 /
 // 46.3, at 32 rows 48.1 / 35.6 against 29.3 / 36.4, its activations being read
@@ -1102,10 +1102,10 @@ constexpr int kSkinnyM = 16;
 // them); a larger weight's few-tile product sums K ranges.
 constexpr int64_t kRangeWeight = 1 << 20;
 bool sums_ranges(int64_t N, int64_t K) { return N * K >= kRangeWeight; }
-constexpr Config kConfigs[12] = {{256, 256, 512, 1, 1.15}, {128, 128, 256, 2, 0.9}, {256, 256, 256, 1, 1.15},
+constexpr Config kConfigs[11] = {{256, 256, 512, 1, 1.15}, {128, 128, 256, 2, 0.9}, {256, 256, 256, 1, 1.15},
                                 {256, 256, 512, 1, 1.0},  {128, 128, 256, 2, 0.1}, {256, 256, 256, 1, 1.3},
                                 {224, 256, 256, 1, 1.2},  {256, 256, 256, 1, 1.25}, {256, 256, 512, 1, 1.3},
-                                {256, 256, 512, 1, 1.3},  {16, 16, 256, 1, 0.1},  {128, 128, 512, 1, 0.6}};
+                                {256, 256, 512, 1, 1.3},  {128, 128, 512, 1, 0.6}};
 
 int64_t tiles_of(const Problem& p, int cfg) {
     const Config c = kConfigs[cfg];
