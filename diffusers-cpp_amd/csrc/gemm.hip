@@ -1098,8 +1098,12 @@ constexpr int kSplitConfig = 10, kSkinnyConfig = 11;
 // again for every 16 weight rows.
 constexpr int kSkinnyM = 16;
 // Weights of fewer elements keep one running sum over ascending k, the order of
-// every configuration a caller can name (C is then the same bits in all of
-// them); a larger weight's few-tile product sums K ranges.
+// every configuration a caller can name: C is then the same bits in all of
+// them, which dt_gemm_bf16_config promises and its callers compare (shapes up to 256 x
+// 3072).  This is that promise's line and not the faster side's: without it 3072 x 256 at
+// one row takes 4.9 us instead of 8.2, 128 x 3072 at 4096 rows 20 instead of 40, 512 x 1536 at
+// 200 rows 14 instead of 23, and none of thirty small products longer.  A larger weight's
+// few-tile product sums K ranges.
 constexpr int64_t kRangeWeight = 1 << 20;
 bool sums_ranges(int64_t N, int64_t K) { return N * K >= kRangeWeight; }
 constexpr Config kConfigs[11] = {{256, 256, 512, 1, 1.15}, {128, 128, 256, 2, 0.9}, {256, 256, 256, 1, 1.15},

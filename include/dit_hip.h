@@ -345,8 +345,15 @@ int dt_gemm_q8_0(const void *A, int64_t lda, const void *codes, int64_t ld_codes
  * Q8_0 weights dequantised as they are staged, 8 = config 5 in eight waves
  * of 128x64 (two per SIMD; the 256x256 kernel dt_gemm_bf16 picks), 9 =
  * config 7 in eight waves (the Q8_0 one); -1 picks by shape as dt_gemm_bf16
- * does (bf16: 8 or 1; Q8_0: 9 or 1).  Every configuration gives the same
- * bits.  For tuning and tests; no counterpart in the reference. */
+ * does: 8 (Q8_0: 9), 1, or, where N * K >= 2^20, one of two that cannot be named:
+ * 128x128 in two groups of waves that each sum every second 64 k (few tiles), and
+ * 16 weight rows per workgroup with a range of K per wave (at most 16 rows).
+ * Configurations 0 to 9, and so -1 for a smaller weight, sum k in the same order and
+ * give the same bits.  The two others, and the K ranges of dt_gemm_bf16_ws, sum in
+ * their own order: C then depends in its last fp32 bits on M, N, K, and on the other
+ * members of a group.  Q8_0 weights and their dequantised bf16 copies take the same one
+ * and give the same bits in every case.  For tuning and tests; no counterpart in the
+ * reference. */
 int dt_gemm_bf16_config(const void *A, int64_t lda, const void *B, int64_t ldb, void *C,
                         int64_t ldc, int64_t M, int64_t N, int64_t K, const float *bias,
                         const void *addend, int64_t ldd, int32_t c_type, int32_t config,

@@ -314,6 +314,24 @@ def test_gemm_few_tiles(orc, dev, M, N, K, weights, out_dtype):
     check(host(out2), lin, out_dtype, f"few tiles grouped {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(1, 257, 4160), (16, 16400, 64), (513, 4100, 320), (250, 3204, 448),  # few rows; two k-groups
+                                   (40, 516, 2112), (130, 2050, 2112)])                           # K ranges
+def test_gemm_q8_0_sum_orders_equal_dequant(orc, dev, M, N, K, out_dtype):
+    """Weights of 2^20 elements and more, whose products take sum orders of their own: a
+    Q8_0 weight and its dequantised copy take the same one, alone and grouped, bit for bit."""
+    print(f"gemm_q8_0 sum orders M={M} N={N} K={K} {out_dtype}", flush=True)
+    assert N * K >= 1 << 20
+    a = dev_tensor(orc.randn(SEED + 278, (M, K)), torch.bfloat16)
+    _, q8, wd = _q8_weight(orc, SEED + 279, N, K)
+    y, y_ref = dit_hip.gemm_q8_0(a, q8, out_dtype=out_dtype), dit_hip.gemm(a, wd, out_dtype=out_dtype)
+    outs = [torch.empty((M, N), dtype=out_dtype, device="cuda") for _ in range(2)]
+    for w, out in zip((q8, wd), outs):
+        dit_hip.gemm_grouped([(a, w, out)])
+    torch.cuda.synchronize()
+    assert torch.equal(y, y_ref) and torch.equal(*outs)
+
+
 def test_prepared_launch_keeps_its_scratch(orc, dev):
     """prepare()'s repeats of calls with scratch of their own (K ranges of a
     product, fp32 attention's parts) after that memory could be given away."""
