@@ -286,11 +286,12 @@ def test_gemm_q8_0_rejects(orc, dev):
 @pytest.mark.parametrize("weights", ["bf16", "q8_0"])
 @pytest.mark.parametrize("M,N,K", [(1, 257, 4160), (16, 4100, 320), (7, 16400, 64),         # few rows, four or eight waves
                                    (17, 5200, 256), (250, 3204, 448), (513, 4100, 320),     # two k-groups, odd k-tiles
-                                   (17, 516, 2112), (300, 253, 4160), (130, 2050, 576)])    # K ranges, ragged
+                                   (17, 516, 2112), (300, 253, 4160), (130, 2050, 1088)])   # K ranges, ragged
 def test_gemm_few_tiles(orc, dev, M, N, K, weights, out_dtype):
     """Products of few rows or few tiles, through gemm / gemm_q8_0 (K ranges with
     a workspace) and the grouped call (none), with bias, addend and strides."""
     print(f"few tiles {weights} {M}x{N}x{K} {out_dtype}", flush=True)
+    assert (dit_hip.load().dt_gemm_bf16_workspace_bytes(M, N, K) > 0) == (M > 16 and K >= 1024)
     a, b = orc.randn(SEED + 270, (M, K + 8)), orc.randn(SEED + 271, (N, K), std=0.02)
     bias, add = orc.randn(SEED + 272, (N,), std=0.1), orc.randn(SEED + 273, (M, N))
     x = dev_tensor(a, torch.bfloat16)[:, :K]
@@ -335,7 +336,9 @@ def test_gemm_q8_0_sum_orders_equal_dequant(orc, dev, M, N, K, out_dtype):
 def test_prepared_launch_keeps_its_scratch(orc, dev):
     """prepare()'s repeats of calls with scratch of their own (K ranges of a
     product, fp32 attention's parts) after that memory could be given away."""
-    a, b = dev_tensor(orc.randn(SEED + 274, (130, 576)), torch.bfloat16), dev_tensor(orc.randn(SEED + 275, (2050, 576)), torch.bfloat16)
+    a, b = dev_tensor(orc.randn(SEED + 274, (130, 2112)), torch.bfloat16), dev_tensor(orc.randn(SEED + 275, (2050, 2112)), torch.bfloat16)
+    assert dit_hip.load().dt_gemm_bf16_workspace_bytes(130, 2050, 2112) > 0
+    assert dit_hip.load().dt_gemm_f32_workspace_bytes(130, 2050, 2112) > 0
     q = dev_tensor(orc.randn(SEED + 276, (1, 70, 2, 128)), torch.float32)
     for fn, args in ((dit_hip.gemm, (a, b)), (dit_hip.gemm_f32, (a.float(), b.float())), (dit_hip.flash_attn_f32, (q, q, q))):
         out, launch = dit_hip.prepare(fn, *args)
@@ -393,13 +396,16 @@ ATTN_SHAPES = [(1, 300, 300, 3), (2, 128, 64, 2), (1, 77, 500, 1), (1, 64, 1, 2)
 
 # ------------------------------------------------------------- fp32 path --
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (130, 200, 320), (256, 256, 3072), (77, 33, 40), (300, 136, 3),
-                                   (129, 260, 12288), (3, 16400, 128), (16, 100, 3072), (32, 68, 176), (17, 130, 2112)])
+                                   (129, 260, 12288), (3, 16400, 128), (16, 100, 3072), (32, 68, 176), (17, 130, 2112),
+                                   (130, 253, 4160)])
 def test_gemm_f32(orc, dev, M, N, K):
     """F32 weights with F32 activations (the reference's own Linear precision)
     in exact bf16 parts, against the oracle's linear at the fp32 bar
     (|d| <= 1e-5 max(|ref|, 1)); with a bias and an addend; K of any size
     (3 and 40 take the masked loads)."""
     print(f"gemm_f32 M={M} N={N} K={K}", flush=True)
+    ranges = M > 32 and K >= 3072  # taken over ranges of K; N = 253: ragged partial rows
+    assert (dit_hip.load().dt_gemm_f32_workspace_bytes(M, N, K) > 0) == ranges
     a = orc.randn(SEED + 280, (M, K))
     b = orc.randn(SEED + 281, (N, K), std=0.02)
     bias = orc.randn(SEED + 282, (N,), std=0.1)
