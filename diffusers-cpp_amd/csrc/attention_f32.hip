@@ -308,7 +308,10 @@ __global__ __launch_bounds__(256, 2) void flash_attn_f32_kernel(const F32Attn a)
         for (int j = 0; j < 3; ++j) qf[j][c] = __builtin_bit_cast(bf16x8_t, p[j]);
     }
     for (int i = tid; i < 2 * a.kv_blocks; i += 256) odd |= a.flags[(int64_t)bh * 2 * a.kv_blocks + i] != 0;
-    if (__syncthreads_or(odd)) {
+    // Marked unlikely: with attn_native in line the compiler put a wait for every DMA in
+    // flight at the top of the key loop (24 heads of 1536 244.5 -> 247.3 us, 2 of 328 26.6 ->
+    // 27.2).  Behind it, it keeps the loop as it was and spills three of attn_native's registers.
+    if (__builtin_expect(__syncthreads_or(odd), 0)) {
         // attn_combine_kernel leaves rows with l = NaN as they are
         if (a.splits > 1 && q < a.seq_q && g == 0)
             a.ml[((int64_t)split * a.bh + bh) * a.seq_q + q] = make_float2(0.f, NAN);
