@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256) void conv2d_kernel(const ConvArgs a) {
 // LDS stages of 16 channels, filled one chunk ahead; eight waves (two per SIMD: one's
 // MFMAs cover the other's LDS reads and waits) of 64 co x 32 FN px (2 x FN MFMA 32x32x16 per tap).
 // Four waves of twice the pixels, one per SIMD, took 160 us instead of 126 at
-// [1,128,512,512] -> 128, 178 instead of 162 at [1,512,160,160] -> 512 and, with the
+// [1,128,512,512] -> 128, 178 instead of 162 at [1,512,160,160] -> 512 (256-pixel tiles) and, with the
 // residual epilogue on 256 pixels, 187 instead of 130 at [1,128,512,512]; the
 // statistics epilogue, which adds its waves' sums in pairs, keeps them.  The DMA source swaps each
 // 32-byte record's two 16-byte units by the rule below (kSwzBit), so
@@ -445,7 +445,7 @@ constexpr int kCi2 = 16, kRec2 = 32;
 // SQ_LDS_IDX_ACTIVE.)
 constexpr int kSwzBit = 3;
 // DMA lanes per X stage: 2 per record, up to the largest patch of the tile
-// shapes conv_geometry2 picks (8 x 32 or 16 x 16 pixels; 16 x 32 or 32 x 16), in
+// shapes of conv_geometry2 (4 x 32 to 16 x 32 pixels, 8 x 16 to 32 x 16), in
 // whole instructions of `threads` lanes.  Lanes past the patch read the zero tail.
 constexpr int conv_patch_lanes(int px, int K) {
     const int wide = (px / 32 + K - 1) * (32 + K - 1), tall = (px / 16 + K - 1) * (16 + K - 1);
@@ -798,12 +798,12 @@ __global__ __launch_bounds__(64 * NWV) void conv2d_dma_kernel(const ConvArgs a, 
 }
 
 // ---- 1x1 on bf16, straight from NCHW --------------------------------------------
-// A 1x1 conv is bound by reading x and writing y ([1, 256, 512, 512] -> 128: 201 MB,
-// 39 us at 5.1 TB/s); through the channel-last copy it read x, wrote and read the copy
-// and took 138 us.  Here the [32 channels][256 pixels] slices of x stream into LDS as
-// they lie, whole 512-byte rows, and the MFMA's pixel operand is read from them
-// transposed (ds_read_tr16_b64: lane i of a 16-lane group gets four channels of pixel
-// i), so x is read once per 128 output channels and nothing else is written.
+// A 1x1 conv is bound by reading x and writing y ([1, 256, 512, 512] -> 128: 201 MB, 39 us at
+// 5.1 TB/s); through the channel-last copy it read x, wrote and read the copy and took 137 us
+// a call in four waves; here 50 (53 in a resnet under the profiler). The [32 channels][256
+// pixels] slices of x stream into LDS as they lie, whole 512-byte rows, and the MFMA's pixel
+// operand is read from them transposed (ds_read_tr16_b64: lane i of a 16-lane group gets four
+// channels of pixel i), so x is read once per 128 output channels and nothing else is written.
 // Eight waves of 64 channels x 64 pixels; three stages of 24 KB, two in flight, and two
 // workgroups per CU.  The channels are summed in the same order as through the
 // copy (k-steps of 16, ascending): the same bits.
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(512, 4) void conv1x1_kernel(const ConvArgs a, int64
     const uint32_t xlds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
     // Both 16-channel steps' pixel operands of one stage.  The wait is in the
     // block; the compiler's own wait before its transposed reads would also drain the stage
-    // in flight (53 instead of 60 us at [1, 256, 512, 512] -> 128, profiled).
+    // in flight (53 instead of 60 us at [1, 256, 512, 512] -> 128, in a resnet under the profiler).
     auto read_x = [&](int stage, bf16x8_t (&xf)[2][FN]) {
         const uint32_t p0 = xlds + stage * kPwStage + xofs[0], p1 = xlds + stage * kPwStage + xofs[1];
         uint2 r[8];
@@ -1033,9 +1033,9 @@ int conv_launch(const void* x, int64_t N, int64_t Ci, int64_t H, int64_t W, cons
     DT_REQUIRE(!gn || (fold->gn_groups > 0 && Ci % fold->gn_groups == 0 && !stats),
                "%s: the GroupNorm fold needs groups dividing the input channels", what);
     // With a workspace 3x3 convs, and 1x1 convs on bf16, take the DMA path
-    // (gfx950, 1x1 [1, 256, 512, 512] -> 128: bf16 49 us direct and 105 us through
-    // the channel-last copy against 217 us staged; fp32 163 us through the copy, reading
-    // twice the bytes, against 136 us staged).
+    // (gfx950, 1x1 [1, 256, 512, 512] -> 128, calls in a loop: bf16 50 us direct and 105 us
+    // through the channel-last copy against 217 us staged; fp32 163 us through the copy,
+    // reading twice the bytes, against 134 us staged).
     const bool dma = conv_uses_dma(K, io_type) && ws && ws_bytes >= (size_t)(nhwc_elems(N, Ci, H, W) * 2 + 256) &&
                      aligned16(ws) && (!stats || (a.cg >= 4 && a.cg <= 64));
     int64_t tiles_w, tiles_h;

@@ -117,9 +117,9 @@ inline bool conv_uses_dma(int64_t K, int32_t io_type) { return K == 3 || (K == 1
 
 // Whether such a conv, without statistics, is a 1x1 on bf16 read straight from
 // NCHW (conv1x1_kernel: whole 32-channel slices of 16-byte pixel groups), without
-// a channel-last copy.  A y that overlaps x keeps the copy, and so do planes under
-// 1024 pixels, where its launch is all there is to win ([1, 256, 16, 20] -> 128 18.7 us
-// against 16.0) and the launches a block reports stay as they were.
+// a channel-last copy.  A y that overlaps x keeps the copy.  So do planes under 1024
+// pixels, not for speed ([1, 256, 16, 20] -> 128 18.7 us against 16.0 without it) but for the
+// number of launches dt_graph_compute reports there, which callers compare.
 inline bool conv_is_direct(int64_t K, int32_t io_type, int32_t upscale2, const void* x, int64_t N, int64_t Ci,
                            int64_t HW, const void* y, int64_t Co) {
     const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
